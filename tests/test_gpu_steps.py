@@ -32,6 +32,29 @@ def test_adaln_tables(dev, R, td, m, C):
     assert bad.size == 0, f"{bad.size} differ, first {bad[:5]}: {got[bad[:5]]} vs {want[bad[:5]]}"
 
 
+@pytest.mark.parametrize("R", [1, 2, 3, 4, 5, 9])
+@pytest.mark.parametrize("td,m,C", [(1, 1, 5), (30, 1, 11), (32, 1, 64), (36, 2, 53), (64, 1, 32), (68, 1, 33), (132, 1, 16),
+                                    (97, 1, 43)])
+def test_adaln_tables_tiles(dev, R, td, m, C):
+    """the edges of the kernel's tiles: one, two, three and more tiles of 32 columns, a last tile cut short, rows of
+    whole 16-byte pieces and not, a last group of fewer than 64 outputs, and one to four timesteps a pass"""
+    test_adaln_tables(dev, R, td, m, C)
+
+
+def test_rotations_wide(dev):
+    """positions from 0 to 1e6 (angles over many turns): the correctly rounded cos and sin of the float32 angle"""
+    g = np.random.default_rng(93)
+    S, n = 1500, 21
+    positions = np.concatenate([np.arange(1500.0)[:600], g.uniform(0, 1e3, 600), 10 ** g.uniform(0, 6, 300)])
+    positions = np.stack([positions, g.permutation(positions), -positions], 1)
+    inv = (1.0 / np.power(np.float32(10000.0), np.arange(n, dtype=np.float32) / np.float32(n))).astype(np.float32)
+    cs = new(dev, "F32", [S, 3 * n, 2])
+    ops.rotations(up(dev, positions, "F64", [S, 3]), up(dev, inv, "F32", [n]), cs)
+    ang = (positions.astype(np.float32)[:, :, None] * inv[None, None, :]).astype(np.float64)
+    cr = np.stack([np.cos(ang), np.sin(ang)], -1).astype(np.float32).ravel()
+    assert np.array_equal(cs.to_numpy().ravel().view(np.int32), cr.view(np.int32))
+
+
 def fixture_request():
     gold = json.load(open(os.path.join(HERE, "golden", "layout_384x288_2s.json")))
     m = {k: int(v) for k, v in gold["metadata"].items() if k != "sigma"}
