@@ -12,7 +12,7 @@ namespace h3 {
 
 // q of Hq heads (row stride qs) and k, v of Hkv heads (row stride kvs) prepared into aq [Hq, Sp, DK], ak [Hkv, Sp, DK]
 // (int8 codes with their scales for SAGE, else half) and av [Hkv, DK, Sp] (half), DK = attn_dk(D), zero past D
-// (q_in_kernel: the pipelined kernel forms q's fragments from q itself, so q is not prepared)
+// (q_in_kernel: the wide kernel forms q's fragments from q itself, so q is not prepared)
 template <int DT>
 static void prep(Ctx* c, const void* q, const void* k, const void* v, int64_t S, int64_t Sp, int64_t Hq, int64_t Hkv, int D,
                  int64_t qs_stride, int64_t kv_stride, bool sage, bool q_in_kernel, int8_t* aq, int8_t* ak, uint16_t* av,
@@ -66,17 +66,18 @@ static int attention_one(Ctx* c, const char* fn, const void* q, const void* k, c
     // the int8 form as the reference takes it (kernels/h3sycl.cpp:1706): heads of 64 or 128 features, and S * D * H
     // within int32; every other call runs the 16-bit form
     const bool sage = !causal && c->sage_want && S >= c->sage_min_s && (D == 64 || D == 128) && S <= INT32_MAX / D / Hq;
-    // heads of 128 features into an aligned out, no causal mask: the pipelined kernel (256 queries a block)
-    const bool pp = !causal && D == 128 && aligned16(out) && S <= (int64_t) kAttnPPTiles * kAttnRows;
+    // heads of 128 features into an aligned out, no causal mask: the wide kernel (256 queries a block)
+    const bool pp = !causal && D == 128 && aligned16(out);
     const int64_t qblock = pp ? kAttnPPQ : kAttnQBlock;
     const int64_t Sp = (S + qblock - 1) / qblock * qblock, nbp = Sp / kAttnRows;
     const int64_t esz = sage ? 1 : 2, DK = attn_dk(D);
     if (Hq * (Sp / qblock) > 0x7fffffff) return fail(std::string(fn) + ": too many query blocks");
-    // the pipelined kernel reads q's rows itself where they are whole 16-byte vectors (no prepared q then)
+    // the wide kernel reads q's rows itself where they are whole 16-byte vectors (no prepared q then)
     const bool q_in_kernel = pp && aligned16(q) && (qs_stride * elem_size(dt)) % 16 == 0;
     int8_t* aq = q_in_kernel ? nullptr : c->scratch<int8_t>(Ctx::ATT_Q, (size_t) (Sp * Hq * DK * esz));
-    int8_t* ak = c->scratch<int8_t>(Ctx::ATT_K, (size_t) (Sp * Hkv * DK * esz));
-    uint16_t* av = c->scratch<uint16_t>(Ctx::ATT_V, (size_t) (Sp * Hkv * DK));
+    const size_t over = pp ? kAttnOver : 0;                   // what its last direct loads read past the end
+    int8_t* ak = c->scratch<int8_t>(Ctx::ATT_K, (size_t) (Sp * Hkv * DK * esz) + over);
+    uint16_t* av = c->scratch<uint16_t>(Ctx::ATT_V, (size_t) (Sp * Hkv * DK) + over / 2);
     float* af = c->scratch<float>(Ctx::ATT_AUX, (size_t) ((Hq + Hkv) * nbp + Hkv * D));
     if ((!aq && !q_in_kernel) || !ak || !av || !af) return -1;
     float *qs = af, *ks = af + Hq * nbp, *km = af + (Hq + Hkv) * nbp;
@@ -101,13 +102,13 @@ static int attention_one(Ctx* c, const char* fn, const void* q, const void* k, c
     P.q_dt = dt;
     const int64_t nblocks = Hq * P.nqb;
     P.nfull = nblocks; P.nsplit = 1; P.ts = 0; P.po = nullptr; P.pml = nullptr;
-    // the pipelined kernel's last round: when it would fill at most half the CUs, its blocks each become up to
+    // the wide kernel's last round: when it would fill at most half the device (two blocks a CU), its blocks each become up to
     // c->attn_split blocks of consecutive key tiles, whose results attn_merge_kernel combines
     int64_t tail = 0;
     if (pp) {
-        const int64_t cus = c->cus, T = (S + kAttnRows - 1) / kAttnRows, last = nblocks % cus;
-        const int64_t want = std::min<int64_t>({(int64_t) c->attn_split, last ? cus / last : 1, T});
-        if (last > 0 && 2 * last <= cus && want > 1) {
+        const int64_t slots = 2 * (int64_t) c->cus, T = (S + kAttnVT - 1) / kAttnVT, last = nblocks % slots;
+        const int64_t want = std::min<int64_t>({(int64_t) c->attn_split, last ? slots / last : 1, T});
+        if (last > 0 && 2 * last <= slots && want > 1) {
             const int64_t ts = (T + want - 1) / want, ns = (T + ts - 1) / ts;
             // (no room for the partial sums under the memory cap: the last round runs unsplit)
             if (ns > 1 && (P.po = c->scratch<float>(Ctx::ATT_PART, (size_t) (last * ns * kAttnPPQ * (128 + 2))))) {
@@ -133,8 +134,8 @@ static int attention_one(Ctx* c, const char* fn, const void* q, const void* k, c
         else H3_ATTN_D(SG, 64, CA)                                                             \
     }
     if (pp) {
-        if (sage) attn_pl_kernel<true, 4><<<grid, 512, 0, c->stream>>>(P);
-        else attn_pl_kernel<false, 4><<<grid, 512, 0, c->stream>>>(P);
+        if (sage) attn_pl_kernel<true, 6><<<grid, 256, 0, c->stream>>>(P);
+        else attn_pl_kernel<false, 4><<<grid, 256, 0, c->stream>>>(P);
         if (tail) attn_merge_kernel<<<(unsigned) ((tail * kAttnPPQ * 32 + 255) / 256), 256, 0, c->stream>>>(P, tail);
     } else if (causal) H3_ATTN(false, true)
     else if (sage) {

@@ -7,10 +7,11 @@
 // divided by the row sum, rounded to half (the reference's result buffer is half) and stored in out's type.
 //
 // Layouts (prepared once per call, in the context's scratch): codes or halves of q and k [H, Sp, DK], v transposed to
-// half [H, DK, Sp] (keys permuted inside each group of 16: attn_vt_pos), Sp = S rounded up to 128 (256 for the
-// pipelined kernel) with zero rows, DK = the head size D rounded up to 64, 128 or 256 with zero
-// features (which change no score and no block max); the output keeps the D features. One block = 4 wavefronts = 128 queries of one head; a
-// wavefront owns 32 queries and walks all keys 64 at a time. Per 64-key tile:
+// half in blocks of 32 keys [H, Sp / 32, DK, 32] (a block is contiguous; keys permuted inside each group of 16:
+// attn_vt_pos), Sp = S rounded up to 128 (256 for the wide kernel) with zero rows, DK = the head size D rounded up to 64,
+// 128 or 256 with zero features (which change no score and no block max); the output keeps the D features. One block = 4
+// wavefronts = 128 queries of one head; a wavefront owns 32 queries and walks all keys 64 at a time (the wide kernel: 64
+// queries, 32 keys). Per 64-key tile:
 //   S^T = K Q^T:  v_mfma_i32_32x32x32_i8 (or f32_32x32x16_f16) with K as the first operand, so every lane ends with
 //                 scores of one query (lane % 32) for 32 of the 64 keys (the other 32 in lane ^ 32);
 //   softmax:      the row max needs one exchange with lane ^ 32 (v_permlane32_swap); the exponents' reference
@@ -38,6 +39,7 @@ constexpr h2_a h2_one = {(_Float16) 1.0f, (_Float16) 1.0f};
 
 constexpr int kAttnRows = 64;            // the reference's scale block (kSageBlock, h3sycl.cpp:1681) and the key tile
 constexpr int kAttnQBlock = 128;         // queries of a block
+constexpr int kAttnVT = 32;              // keys of a block of the prepared v^T, and of a key tile of the wide kernel
 constexpr int kAttnMaxD = 256;           // the largest head: heads of D features run in kernels of 64, 128 or 256
 // the kernel head size of a head of D features (D <= kAttnMaxD)
 inline int attn_dk(int64_t D) { return D <= 64 ? 64 : D <= 128 ? 128 : 256; }
@@ -66,6 +68,17 @@ __device__ __forceinline__ uint16_t half_bits(float x) {
 __device__ __forceinline__ void attn_dma16(const void* g, const void* lds_dst) {
     const uint32_t m = (uint32_t) (uintptr_t) lds_dst;
     asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(m) : "memory", "m0");
+}
+// the same from a wave-uniform base and a 32-bit lane offset; N = 2: a second load 1024 bytes further in both places (the
+// instruction's offset counts for the LDS address too)
+template <int N>
+__device__ __forceinline__ void attn_dma16s(const void* base, uint32_t off, uint32_t lds_dst) {
+    static_assert(N == 1 || N == 2, "attn_dma16s");
+    if constexpr (N == 1)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_dst) : "memory", "m0");
+    else
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024"
+                     ::"v"(off), "s"(base), "s"(lds_dst) : "memory", "m0");
 }
 #pragma clang diagnostic pop
 
@@ -362,9 +375,9 @@ __global__ __launch_bounds__(256) void attn_v_prep_vec_kernel(const void* __rest
     // 16 g + 4 e + (0..3) then 16 g + 8 + 4 e + (0..3)
 #pragma unroll
     for (int k = 0; k < D * 8 / 256; ++k) {
-        const int u = tid + 256 * k, d = u / 8, c = u % 8, t = 16 * (c / 2) + 4 * (c % 2);
+        const int u = tid + 256 * k, half = u / (4 * D), d = u / 4 % D, c = 4 * half + u % 4, t = 16 * (c / 2) + 4 * (c % 2);
         const uint32_t* row = reinterpret_cast<const uint32_t*>(tile + d * PITCH + t);
-        *reinterpret_cast<uint4*>(vt + (h * D + d) * Sp + t0 + 8 * c) = make_uint4(row[0], row[1], row[4], row[5]);
+        *reinterpret_cast<uint4*>(vt + (h * Sp + t0) * D + 8 * u) = make_uint4(row[0], row[1], row[4], row[5]);
     }
 }
 
@@ -381,8 +394,8 @@ __global__ __launch_bounds__(256) void attn_v_prep_kernel(const void* __restrict
     }
     __syncthreads();
     for (int e = tid; e < n; e += 256) {
-        const int d = e / kAttnRows, t = e % kAttnRows;
-        vt[(h * DK + d) * Sp + t0 + attn_vt_pos(t)] = tile[t * pitch + d];
+        const int t = e % kAttnVT + e / (kAttnVT * DK) * kAttnVT, d = e / kAttnVT % DK;
+        vt[(h * Sp + t0 + t / kAttnVT * kAttnVT) * DK + d * kAttnVT + attn_vt_pos(t % kAttnVT)] = tile[t * pitch + d];
     }
 }
 
@@ -393,6 +406,9 @@ __device__ __forceinline__ uint32_t attn_pack_h2(float a, float b) {
     const f2 v = {a, b};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, h2_a));
 }
+
+// a workgroup barrier without waits: what has to be complete is waited for before it
+__device__ __forceinline__ void block_barrier_a() { asm volatile("s_barrier" ::: "memory"); }
 
 // ---- the attention kernel ----
 struct AttnArgs {
@@ -406,17 +422,17 @@ struct AttnArgs {
     void* out;                // [S, H * D]
     int out_dt;
     int D;                    // the heads' features (the kernel's DK of them are prepared, zero past D)
-    int nqb;                  // query blocks per head (of 128 queries, or 256 in the pipelined kernel)
+    int nqb;                  // query blocks per head (of 128 queries, or 256 in the wide kernel)
     int kvdiv;                // query heads per key/value head: head h reads k and v of head h / kvdiv
     int64_t Spk;              // rows of the prepared k and v^T (Sp unless they come from another sequence)
-    // the pipelined kernel's split of the last round: blocks [nfull, nfull + tail * nsplit) each take key tiles
+    // the wide kernel's split of the last round: blocks [nfull, nfull + tail * nsplit) each take key tiles
     // [s ts, s ts + ts) of query block nfull + (b - nfull) / nsplit (s = (b - nfull) % nsplit) and leave O, m and l
     // in po / pml for attn_merge_kernel; nfull = the grid and nsplit = 1 when nothing is split
     int64_t nfull;
     int nsplit, ts;
     float* po;                // [tail * nsplit, 256, DK] O before the division by l
     float* pml;               // [tail * nsplit, 256, 2] m and l
-    // the pipelined kernel with qraw set reads q from the caller's rows (stride qstride elements of type q_dt, 16-byte
+    // the wide kernel with qraw set reads q from the caller's rows (stride qstride elements of type q_dt, 16-byte
     // aligned) and forms its fragments itself, as attn_qk_prep_vec_kernel would (q and qs are then unused)
     const void* qraw;
     int64_t qstride;
@@ -483,7 +499,7 @@ __global__ __launch_bounds__(256, DK == 256 ? 1 : 3) void attn_kernel(AttnArgs P
 #pragma unroll
         for (int j = 0; j < VI; ++j) {
             const int i = wave * VI + j, u = 64 * i + lane, r = u / 8, c = attn_swz<8>(r, u % 8);
-            const uint16_t* gv = vbase + (int64_t) r * Spk + (int64_t) t * kAttnRows + 8 * c;
+            const uint16_t* gv = vbase + (((int64_t) t * 2 + c / 4) * DK + r) * kAttnVT + 8 * (c % 4);
             __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*) gv,
                                              (__attribute__((address_space(3))) void*) (s + KTB + 1024 * i), 16, 0, 0);
         }
@@ -645,37 +661,43 @@ __global__ __launch_bounds__(256, DK == 256 ? 1 : 3) void attn_kernel(AttnArgs P
 
 
 
-constexpr int kAttnPPQ = 256;            // queries of a pipelined block
+constexpr int kAttnPPQ = 256;            // queries of a wide block
+constexpr size_t kAttnOver = 65536;      // bytes after the prepared k and v^T that its last direct loads may read
 // 1.5 2^23: for |n| < 2^22 the float kScoreBias + n has the bits kScoreBiasBits + n, so int32 score products started
 // from kScoreBiasBits read as floats without a conversion; |score| <= 128 127^2 < 2^22 for heads of 128 features
 constexpr float kScoreBias = 12582912.0f;
 constexpr int kScoreBiasBits = 0x4B400000;
-constexpr int kAttnPPTiles = 4096;       // key tiles it takes (sequences of up to 262144 tokens)
 
 
-// ---- the pipelined form: heads of 128 features, no mask but the sequence's end (both forms) ----
-// One block = 8 wavefronts = 256 queries of one head, 32 a wavefront as above, two wavefronts a SIMD. Each step a
-// wavefront computes the scores of key tile t + 1, then tile t's P v products with the softmax of tile t + 1 (the
-// two are independent) between them: a wavefront issues a few VALU instructions between its own matrix products at
-// no cost to them, and both wavefronts of a SIMD do so. One workgroup barrier a step.
-// Key tile j is read in steps j - 1 (its K) and j (its V^T); a ring of NS stages holds it; its stage is refilled
-// (tile j + NS) at the start of step j + 1, every wavefront issuing its share of the direct loads, which it waits for
-// before the barrier that publishes them. The ring's loads are inline asm (attn_dma16), the head's k scales are
-// copied into LDS once, and the int8 score products start from kScoreBias's bits: see the helpers above.
+// ---- the wide form: heads of 128 features, no mask but the sequence's end (both forms) ----
+// Bound by the power the card allows in long sequences (the clock falls to 1.8-2.0 GHz), by the issue of each
+// wavefront's own instructions in short ones. One block = 4 wavefronts = 256 queries of one head; a wavefront owns 64 queries
+// (two groups of 32) and walks the keys 32 at a time: a fragment of K or V^T read from LDS feeds two products, half the
+// LDS reads a product of one group a wavefront, which ran at 1.80 instead of 2.0 GHz under the same power. Two blocks a CU: the
+// two wavefronts of a SIMD belong to different blocks, with no barrier between them, so one's softmax runs beside the
+// other's products. Per tile: the softmax of both groups, a barrier, then the P v products and the next tile's scores
+// back to back at a raised issue priority, with the ring's refill and the next fragments' reads between them.
+// 56 heads: 47104 tokens 44.4 -> 41.5 ms, 2159 tokens (16-bit form) 174 -> 155 us for the whole call. Others tried: three blocks a CU of one group
+// a wavefront, 14 % fewer cycles but at 1.62 GHz (43.7 ms); eight wavefronts sharing one ring, 42.4 ms, 42.2 with
+// their barriers half a tile apart; products and softmax taking turns behind barriers, 45.4 ms.
+// A ring of NS stages holds the key tiles; the stage of tile t - 1 is refilled with tile t + NS - 1 after the barrier
+// inside tile t's step, every wavefront issuing its share of the direct loads, which it waits for before the barrier that
+// publishes them (the one inside the step of the tile before). The ring's loads are inline asm (attn_dma16s), and the
+// int8 score products start from kScoreBias's bits: see the helpers above.
 // A block of a split last round (AttnArgs::nfull) walks only its range of key tiles, counted from its first, and
 // leaves O, m and l to attn_merge_kernel.
 template <bool SAGE, int NS>
-__global__ __launch_bounds__(512, 1) void attn_pl_kernel(AttnArgs P) {
-    constexpr int DK = 128, ESZ = SAGE ? 1 : 2, RB = DK * ESZ, CPR = RB / 16, NQF = RB / 32;
-    constexpr int KTB = kAttnRows * RB, VTB = DK * kAttnRows * 2, STAGE = KTB + VTB;
+__global__ __launch_bounds__(256, 2) void attn_pl_kernel(AttnArgs P) {
+    constexpr int DK = 128, ESZ = SAGE ? 1 : 2, RB = DK * ESZ, CPR = RB / 16, NQF = RB / 32, NG = 2;
+    constexpr int KTB = kAttnVT * RB, VTB = DK * kAttnVT * 2, STAGE = KTB + VTB;
     constexpr int NDT = DK / 32;
-    constexpr int KI = KTB / 1024 / 8, VI = VTB / 1024 / 8;   // direct loads of a wavefront a tile (K, V^T)
-    constexpr int LATER = (NS - 3) * (KI + VI);                // loads of later tiles in flight at a tile's wait
-    static_assert(NS >= 3 && KI >= 1 && VI >= 1, "ring");
-    __shared__ __attribute__((aligned(16))) int8_t lds[NS * STAGE];
-    // SAGE: the key tiles' scales of the head, copied once (a global load in the loop would sit behind the ring's
-    // direct loads in the same wait counter)
-    __shared__ float ksl[SAGE ? kAttnPPTiles : 1];
+    constexpr int KI = KTB / 1024 / 4, VI = VTB / 1024 / 4, L = KI + VI;   // direct loads of a wavefront a tile
+    static_assert(STAGE % 256 == 0 && KTB % 256 == 0, "the swizzle's XOR of addresses");
+    static_assert(NS >= 3 && KI >= 1 && VI == 2 && (NS - 1) * VTB <= (int) kAttnOver && KTB <= VTB, "ring");
+    // the 16-bit form's q takes twice the registers: each group's last NQL fragments stay in LDS, read as they are used
+    constexpr int NQL = SAGE ? 0 : 2, NQR = NQF - NQL;
+    __shared__ __attribute__((aligned(1024))) int8_t lds[NS * STAGE];
+    __shared__ __attribute__((aligned(16))) v4i_a qlds[NQL ? 4 * NG * NQL * 64 : 1];
     const int tid = threadIdx.x, lane = tid & 63, hl = lane >> 5, ql = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // blocks go to the 8 XCDs round robin: renumbered so that each XCD takes a contiguous run (the blocks of few
@@ -684,7 +706,7 @@ __global__ __launch_bounds__(512, 1) void attn_pl_kernel(AttnArgs P) {
     int b = (int) blockIdx.x;
     // a block of the split last round: its query block and its range of key tiles (slot: its partial sums)
     int slot = -1, t0 = 0;
-    const int nfull = (int) P.nfull, Tall = (int) ((P.S + kAttnRows - 1) / kAttnRows);
+    const int nfull = (int) P.nfull, Tall = (int) ((P.S + kAttnVT - 1) / kAttnVT);
     int T = Tall;
     if (b < nfull) {
         if (nfull % 8 == 0) b = (b % 8) * (nfull / 8) + b / 8;
@@ -694,344 +716,338 @@ __global__ __launch_bounds__(512, 1) void attn_pl_kernel(AttnArgs P) {
         t0 = (slot % P.nsplit) * P.ts;
         T = Tall - t0 < P.ts ? Tall - t0 : P.ts;
     }
+    b = __builtin_amdgcn_readfirstlane(b);
+    t0 = __builtin_amdgcn_readfirstlane(t0);
+    T = __builtin_amdgcn_readfirstlane(T);
     const int64_t h = b / P.nqb, qb = b % P.nqb, Sp = P.Sp, S = P.S;
-    const int64_t q0 = qb * kAttnPPQ + 32 * wave;             // this wavefront's first query
+    const int64_t q0 = qb * kAttnPPQ + 64 * wave;             // this wavefront's first query
     const int64_t nbp = Sp / kAttnRows;
 
-    v4i_a qf[NQF];
+    v4i_a qf[NG][NQF];
+    v4i_a* const qmine = qlds + (SAGE ? 0 : wave * NG * NQL * 64 + lane);   // this lane's [NG][NQL] fragments, 64 apart
     float fq = P.c;
-    // With P.qraw: this lane's 64 features of its query straight from the caller's rows (fragment kk: FR features from
-    // 32 kk + 16 hl for int8 codes, 16 kk + 8 hl for halves), turned into the fragments attn_qk_prep_vec_kernel would
-    // have written: halves here; int8 codes after the prologue's barrier, where the two wavefronts of a 64-row scale
-    // block (wavefronts 2j, 2j + 1) have each left their 32 rows' max in qmax. Rows past S are zeros.
+    // With P.qraw: this lane's 64 features of its two queries straight from the caller's rows (fragment kk: FR features
+    // from 32 kk + 16 hl for int8 codes, 16 kk + 8 hl for halves), turned into the fragments attn_qk_prep_vec_kernel
+    // would have written. The wavefront's 64 queries are one 64-row scale block. Rows past S are zeros.
     constexpr int FR = SAGE ? 16 : 8;
-    __shared__ float qmax[8];
-    float qx[NQF * FR];
-    float qm = 0.0f;
     if (P.qraw) {
-        const int64_t qi = q0 + ql;
-        const int qes = P.q_dt == H3S_F32 ? 4 : 2;
-        const char* qrow = reinterpret_cast<const char*>(P.qraw) + (qi * P.qstride + h * DK) * qes;
+        float qx[NG][NQF * FR];
+        auto qload = [&](auto dt_tag) {
+            constexpr int QDT = decltype(dt_tag)::value, qes = QDT == H3S_F32 ? 4 : 2, QV = 16 / qes;
 #pragma unroll
-        for (int kk = 0; kk < NQF; ++kk) {
-            const int f0 = SAGE ? 32 * kk + 16 * hl : 16 * kk + 8 * hl;
+            for (int gq = 0; gq < NG; ++gq) {
+                const int64_t qi = q0 + 32 * gq + ql;
+                const char* qrow = reinterpret_cast<const char*>(P.qraw) + ((qi < S ? qi : S - 1) * P.qstride + h * DK) * qes;
+                uint4 raw[NQF * FR / QV];
 #pragma unroll
-            for (int c8 = 0; c8 < FR; c8 += 8) {
-                float* x = qx + kk * FR + c8;
-                if (qi >= S) {
+                for (int c = 0; c < NQF * FR / QV; ++c) {
+                    const int e = c * QV, f0 = SAGE ? 32 * (e / FR) + 16 * hl : 16 * (e / FR) + 8 * hl;
+                    raw[c] = *reinterpret_cast<const uint4*>(qrow + (f0 + e % FR) * qes);
+                }
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) x[e] = 0.0f;
-                } else if (P.q_dt == H3S_F32) {
-                    const float4 a = *reinterpret_cast<const float4*>(qrow + (f0 + c8) * 4);
-                    const float4 b = *reinterpret_cast<const float4*>(qrow + (f0 + c8) * 4 + 16);
-                    x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
-                } else {
-                    const uint4 u = *reinterpret_cast<const uint4*>(qrow + (f0 + c8) * 2);
-                    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+                for (int c = 0; c < NQF * FR / QV; ++c) {
+                    float x[QV];
+                    Vec<QDT>::unpack(raw[c], x);
+#pragma unroll
+                    for (int e = 0; e < QV; ++e) qx[gq][c * QV + e] = qi < S ? x[e] : 0.0f;
+                }
+            }
+        };
+        if (P.q_dt == H3S_BF16) qload(std::integral_constant<int, H3S_BF16>{});
+        else if (P.q_dt == H3S_F16) qload(std::integral_constant<int, H3S_F16>{});
+        else qload(std::integral_constant<int, H3S_F32>{});
+        if constexpr (SAGE) {
+            // q's codes (attn_qk_prep_vec_kernel's arithmetic)
+            float qm = 0.0f;
+#pragma unroll
+            for (int gq = 0; gq < NG; ++gq)
+#pragma unroll
+                for (int i = 0; i < NQF * FR; ++i) qm = fmaxf(qm, fabsf(qx[gq][i]));
+            qm = wave_max<64>(qm);
+            const float inv = qm > 0.0f ? 127.0f / qm : 0.0f;
+#pragma unroll
+            for (int gq = 0; gq < NG; ++gq)
+#pragma unroll
+                for (int kk = 0; kk < NQF; ++kk) {
+                    v4i_a w;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        x[2 * i] = P.q_dt == H3S_BF16 ? bf16_lo(w[i]) : f16_lo(w[i]);
-                        x[2 * i + 1] = P.q_dt == H3S_BF16 ? bf16_hi(w[i]) : f16_hi(w[i]);
-                    }
-                }
-            }
-        }
-        if constexpr (SAGE) {
+                        uint32_t b = 0;
 #pragma unroll
-            for (int i = 0; i < NQF * FR; ++i) qm = fmaxf(qm, fabsf(qx[i]));
-            qm = wave_max<64>(qm);
-            if (lane == 0) qmax[wave] = qm;
+                        for (int e = 0; e < 4; ++e) {
+                            const float cc = fminf(fmaxf(roundf(qx[gq][kk * FR + 4 * i + e] * inv), -127.0f), 127.0f);
+                            b |= (uint32_t) ((int) cc & 255) << (8 * e);
+                        }
+                        w[i] = (int) b;
+                    }
+                    qf[gq][kk] = w;
+                }
+            fq = qm / 127.0f * P.c;
         } else {
 #pragma unroll
-            for (int kk = 0; kk < NQF; ++kk) {
-                v4i_a w;
+            for (int gq = 0; gq < NG; ++gq)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) w[i] = (int) pack_f16(qx[kk * FR + 2 * i], qx[kk * FR + 2 * i + 1]);
-                qf[kk] = w;
-            }
+                for (int kk = 0; kk < NQF; ++kk) {
+                    v4i_a w;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) w[i] = (int) pack_f16(qx[gq][kk * FR + 2 * i], qx[gq][kk * FR + 2 * i + 1]);
+                    qf[gq][kk] = w;
+                }
         }
     } else {
-        const int8_t* qrow = P.q + ((h * Sp + q0 + ql) * DK) * ESZ;
 #pragma unroll
-        for (int kk = 0; kk < NQF; ++kk) qf[kk] = *reinterpret_cast<const v4i_a*>(qrow + 32 * kk + 16 * hl);
+        for (int gq = 0; gq < NG; ++gq) {
+            const int8_t* qrow = P.q + ((h * Sp + q0 + 32 * gq + ql) * DK) * ESZ;
+#pragma unroll
+            for (int kk = 0; kk < NQF; ++kk) qf[gq][kk] = *reinterpret_cast<const v4i_a*>(qrow + 32 * kk + 16 * hl);
+        }
         if constexpr (SAGE) fq = P.qs[h * nbp + q0 / kAttnRows] * P.c;
     }
+#pragma unroll
+    for (int gq = 0; gq < NG; ++gq)
+#pragma unroll
+        for (int i = 0; i < NQL; ++i) qmine[(gq * NQL + i) * 64] = qf[gq][NQR + i];
+    if constexpr (SAGE) fq = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(fq)));   // one value a wavefront
 
     const int64_t g = h / P.kvdiv, Spk = P.Spk;
-    if constexpr (SAGE)
-        for (int i = tid; i < T; i += 512) ksl[i] = P.ks[g * nbp + t0 + i];
-    // tiles are counted from t0 (this block's first key tile) from here on
-    const int8_t* kbase = P.k + (g * Spk + (int64_t) t0 * kAttnRows) * RB;
-    const uint16_t* vbase = P.vt + g * DK * Spk + (int64_t) t0 * kAttnRows;
-    // tile t into stage t % NS; a tile past the last loads the last one again (into a stage no tile uses then), so
-    // that every wavefront has the same loads in flight at every wait
-    auto issue = [&](int t) {
-        const int64_t tc = t < T ? t : T - 1;
-        int8_t* s = lds + (t % NS) * STAGE;
+    // k's scales through the scalar cache (constant address space: the kernel writes none of them), a tile ahead
+    typedef const __attribute__((address_space(4))) float* cfloat;
+    const cfloat ksc = (cfloat) wave_uniform(reinterpret_cast<int64_t>(P.ks) + (SAGE ? 4 * g * nbp : 0));
+    // tiles are counted from t0 (this block's first key tile) from here on; a tile's K rows and v^T block are contiguous
+    const int8_t* kbase = reinterpret_cast<const int8_t*>(wave_uniform(reinterpret_cast<int64_t>(P.k) + (g * Spk + (int64_t) t0 * kAttnVT) * RB));
+    const int8_t* vbase = reinterpret_cast<const int8_t*>(
+        wave_uniform(reinterpret_cast<int64_t>(P.vt) + (g * Spk + (int64_t) t0 * kAttnVT) * DK * 2 + wave * VI * 1024));
+    // this lane's place in its direct loads: unit u of a tile (16 bytes) is row u / CPR, chunk swz(u % CPR). The v^T rows
+    // (4 chunks) of a wavefront's loads are 16 apart, where the swizzle repeats: one offset serves them all.
+    uint32_t kvo[KI];
 #pragma unroll
-        for (int j = 0; j < KI; ++j) {
-            const int i = wave * KI + j, u = 64 * i + lane, r = u / CPR, c = attn_swz<CPR>(r, u % CPR);
-            const int8_t* gk = kbase + (tc * kAttnRows + r) * RB + 16 * c;
-            attn_dma16(gk, s + 1024 * i);
-        }
+    for (int j = 0; j < KI; ++j) {
+        const int u = 64 * (wave * KI + j) + lane, r = u / CPR;
+        kvo[j] = (uint32_t) (r * RB + 16 * attn_swz<CPR>(r, u % CPR));
+    }
+    const uint32_t vvo = (uint32_t) ((lane / 4) * 64 + 16 * attn_swz<4>(lane / 4, lane % 4));
+    // The next tile to load, into the stage at byte offset st of the ring. Tiles past the last (into stages no tile uses
+    // then) load what follows it in the scratch, which has room for them, so that every wavefront has the same loads in
+    // flight at every wait.
+    const uint32_t lds0 = (uint32_t) (uintptr_t) lds;
+    auto issue = [&](int st) {
+        const uint32_t dst = lds0 + st;
 #pragma unroll
-        for (int j = 0; j < VI; ++j) {
-            const int i = wave * VI + j, u = 64 * i + lane, r = u / 8, c = attn_swz<8>(r, u % 8);
-            const uint16_t* gv = vbase + (int64_t) r * Spk + tc * kAttnRows + 8 * c;
-            attn_dma16(gv, s + KTB + 1024 * i);
-        }
+        for (int j = 0; j < KI; ++j) attn_dma16s<1>(kbase, kvo[j], dst + 1024 * (wave * KI + j));
+        attn_dma16s<VI>(vbase, vvo, dst + KTB + 1024 * (wave * VI));
+        kbase += KTB;
+        vbase += VTB;
     };
+    auto after = [&](int st) { return st + STAGE == NS * STAGE ? 0 : st + STAGE; };
 
-    v16f_a o[NDT];
+    v16f_a o[NG][NDT];
 #pragma unroll
-    for (int i = 0; i < NDT; ++i) o[i] = (v16f_a) 0.0f;
-    float m = -INFINITY, l = 0.0f;
+    for (int gq = 0; gq < NG; ++gq)
+#pragma unroll
+        for (int i = 0; i < NDT; ++i) o[gq][i] = (v16f_a) 0.0f;
+    float m[NG] = {-INFINITY, -INFINITY}, l[NG] = {0.0f, 0.0f};
     typedef typename std::conditional<SAGE, v16i_a, v16f_a>::type score_t;
-    score_t sc[2];                                             // the scores of the next tile, two 32-key halves
-    v8h_a pb[4];                                               // the weights of the tile whose P v products run now
-    v8h_a pn[4];                                               // the weights being formed for the next tile
+    float ks_next = SAGE ? ksc[t0 / 2] : 0.0f;
 
-    // the scores of tile t + 1 (K of its stage), two 32-key halves, started from kScoreBias's bits (SAGE)
-    auto scores = [&](int t) {
-        const int8_t* sk = lds + ((t + 1) % NS) * STAGE;
+    // K's fragments of a tile (each feeds both groups): the first KP read behind the P v products of the tile before, the
+    // others into their registers as they are used
+    constexpr int KP = SAGE ? 4 : 2;
+    v4i_a kf[KP];
+    // (chunk 2 u + hl of a row is chunk hl's place with bits of u flipped, stages and tiles being whole rows of the swizzle)
+    const uint32_t ka = lds0 + (ql * CPR + attn_swz<CPR>(ql, hl)) * 16, va = lds0 + KTB + (ql * 4 + attn_swz<4>(ql, hl)) * 16;
+    auto kread = [&](int st, int u) {
+        kf[u % KP] = *(const __attribute__((address_space(3))) v4i_a*) (((ka + st) ^ (32 * u)));
+    };
+    v8h_a vf[2][NDT];                                          // V^T's fragments of a 16-key slice
+    int prev = (NS - 1) * STAGE, cur = 0;                      // the stages of tiles t - 1 (refilled with t + NS - 1) and t
+    auto step = [&](int t, auto tail_tag) {
+        constexpr bool TAIL = decltype(tail_tag)::value;
+        const float f = SAGE ? fq * ks_next : fq;
+        const int next = after(cur);
+        // ---- scores: both groups' products of each K fragment, started from kScoreBias's bits (SAGE) ----
+        score_t sc[NG];
         sc[0] = sc[1] = SAGE ? (score_t) kScoreBiasBits : (score_t) 0;
-        v4i_a kf[2][2];
-        auto kread = [&](int u, v4i_a (&d)[2]) {
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int r = 32 * j + ql;
-                d[j] = *reinterpret_cast<const v4i_a*>(sk + (r * CPR + attn_swz<CPR>(r, 2 * u + hl)) * 16);
-            }
-        };
-        kread(0, kf[0]);
 #pragma unroll
         for (int u = 0; u < NQF; ++u) {
-            // the next sub-step's two K fragments read ahead of this one's products, fenced (the scheduler sinks
-            // each read to its product otherwise, and its latency comes before the product)
-            if (u + 1 < NQF) kread(u + 1, kf[(u + 1) & 1]);
-            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                if constexpr (SAGE) sc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[u & 1][j], qf[u], sc[j], 0, 0, 0);
-                else sc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h_a, kf[u & 1][j]),
-                                                                     __builtin_bit_cast(v8h_a, qf[u]), sc[j], 0, 0, 0);
+            for (int gq = 0; gq < NG; ++gq) {
+                const v4i_a qv = u < NQR ? qf[gq][u] : qmine[(gq * NQL + u - NQR) * 64];
+                if constexpr (SAGE) sc[gq] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[u % KP], qv, sc[gq], 0, 0, 0);
+                else sc[gq] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h_a, kf[u % KP]),
+                                                                     __builtin_bit_cast(v8h_a, qv), sc[gq], 0, 0, 0);
             }
-            __builtin_amdgcn_sched_barrier(0);
+            if (u + KP < NQF) kread(cur, u + KP);
         }
-    };
-    // O += P_t v_t: 16 products (V^T of tile t's stage)
-    auto pv = [&](int t) {
-        const int8_t* sv = lds + (t % NS) * STAGE + KTB;
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+        // ---- softmax -> the half weights (pb), the running reference and row sum ----
+        // register i holds key 8 (i / 4) + 4 hl + i % 4 of the tile. SAGE: its bits are those of the float kScoreBias +
+        // score, read as they are.
+        const int lim = (int) (S - (int64_t) (t0 + t) * kAttnVT) - 4 * hl;
+        auto live = [&](int i) { return 8 * (i / 4) + i % 4 < lim; };
+        v8h_a pb[NG][2];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            v4i_a vf[NDT];
+        for (int gq = 0; gq < NG; ++gq) {
+            // the whole vector reinterpreted (an element-wise __builtin_bit_cast(float, sc[i]) compiled to copies of
+            // element 0 here)
+            const v16f_a x = SAGE ? __builtin_bit_cast(v16f_a, sc[gq]) : __builtin_convertvector(sc[gq], v16f_a);
+            // The weights p = 2^(score f - m) rounded to half, packed as the P v products take them (chunk s: registers
+            // 8 s .. 8 s + 7), and their sum over this lane's keys. SAGE: score f - m = x f - (kScoreBias f + m), with
+            // one rounding of the offset (relative 2^-24 of kScoreBias f, far below half's rounding of p).
+            auto weights = [&]() {
+                const float c = SAGE ? __builtin_fmaf(kScoreBias, f, m[gq]) : m[gq];
+                float ls[2];
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    float p[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[8 * s + e], f, -c));
+                        if (TAIL && !live(8 * s + e)) p[e] = 0.0f;
+                    }
+                    const uint32_t a0 = attn_pack_h2(p[0], p[1]), a1 = attn_pack_h2(p[2], p[3]);
+                    const uint32_t b0 = attn_pack_h2(p[4], p[5]), b1 = attn_pack_h2(p[6], p[7]);
+                    ls[s] = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2_a, a0), h2_one, 0.0f, false);
+                    ls[s] = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2_a, a1), h2_one, ls[s], false);
+                    ls[s] = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2_a, b0), h2_one, ls[s], false);
+                    ls[s] = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2_a, b1), h2_one, ls[s], false);
+                    v4i_a pf;                                  // as they are (attn_vt_pos)
+                    pf[0] = (int) a0; pf[1] = (int) a1; pf[2] = (int) b0; pf[3] = (int) b1;
+                    pb[gq][s] = __builtin_bit_cast(v8h_a, pf);
+                }
+                return ls[0] + ls[1];
+            };
+            // First against the current reference m, with no max: a weight past half's range (a score more than about
+            // 16 above m, or m not yet set) rounds to infinity and makes the lane's sum infinite. Only then the tile's
+            // max: m moves when it passes m by more than 8 (as in attn_kernel), O and l are rescaled and the weights
+            // computed again (each at most 1 then). O / l does not depend on m.
+            float lt = weights();
+            if (__any(!(lt <= 3.0e38f))) {
+                asm volatile("" ::: "memory");
+                float mt[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float u = TAIL && !live(i) ? -INFINITY : x[i], w = TAIL && !live(i + 8) ? -INFINITY : x[i + 8];
+                    mt[i] = fmaxf(u, w);
+                }
+#pragma unroll
+                for (int w = 4; w >= 1; w /= 2)
+#pragma unroll
+                    for (int i = 0; i < w; ++i) mt[i] = fmaxf(mt[i], mt[i + w]);
+                const float mx = (attn_pair_max(mt[0]) - (SAGE ? kScoreBias : 0.0f)) * f;
+                if (mx > m[gq] + 8.0f) {
+                    const float mn = fmaxf(m[gq], mx);
+                    const float alpha = __builtin_amdgcn_exp2f(m[gq] - mn);
+                    m[gq] = mn;
+                    l[gq] = l[gq] * alpha;
+#pragma unroll
+                    for (int dt = 0; dt < NDT; ++dt) o[gq][dt] = o[gq][dt] * alpha;
+                }
+                lt = weights();
+            }
+            l[gq] = l[gq] + lt;
+            // slice gq's fragments of V^T, into the registers this group's scores leave
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt) {
-                const int r = 32 * dt + ql;
-                vf[dt] = *reinterpret_cast<const v4i_a*>(sv + (r * 8 + attn_swz<8>(r, 2 * u + hl)) * 16);
+                vf[gq][dt] = *(const __attribute__((address_space(3))) v8h_a*) (((va + cur) ^ (32 * gq)) + 2048 * dt);
             }
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt)
-                o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h_a, vf[dt]), pb[u], o[dt], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
-    };
-    // the softmax of the scores of tile t + 1 -> its half weights (pn), the running max and row sum; sets alpha when
-    // O is to be rescaled (after this step's P v products, which use the old reference)
-    auto softmax = [&](int t, auto tail_tag, float& alpha) {
-        constexpr bool TAIL = decltype(tail_tag)::value;
-        const int tn = t + 1;
-        // register i holds key 64 tn + 32 (i / 16) + 8 ((i % 16) / 4) + 4 hl + i % 4. SAGE: its bits are those of
-        // the float kScoreBias + score (the score products start from kScoreBias's bits), read as they are.
-        float x[32];
+        wait_vm<(NS - 3) * L>();                               // this wavefront's loads of tile t + 1 are in
+        block_barrier_a();                                     // every wavefront's; and every one is done with tile t - 1
+        // ---- O^T += V^T P^T: both groups' products of each V^T fragment; between them the refill of tile t - 1's stage
+        // and the next tile's K fragments and scale ----
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            // the whole vector reinterpreted (an element-wise __builtin_bit_cast(float, sc[j][i]) compiled to copies
-            // of element 0 here)
-            const v16f_a xf = SAGE ? __builtin_bit_cast(v16f_a, sc[j]) : __builtin_convertvector(sc[j], v16f_a);
+        for (int s = 0; s < 2; ++s)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) x[16 * j + i] = xf[i];
-        }
-        const float f = SAGE ? fq * ksl[tn] : fq;
-        const int lim = (int) (S - (int64_t) (t0 + tn) * kAttnRows) - 4 * hl;
-        auto live = [&](int i) { return 32 * (i / 16) + 8 * ((i % 16) / 4) + i % 4 < lim; };
-        // The weights p = 2^(score f - m) rounded to half, packed into pb as the P v products take them, and their
-        // sum over this lane's keys. SAGE: score f - m = x f - (kScoreBias f + m), with one rounding of the offset
-        // (relative 2^-24 of kScoreBias f, far below half's rounding of p).
-        // chunk s: the weights of registers 8 s .. 8 s + 7 into pn[s], their sum
-        auto chunk = [&](int s, float c) {
-                float p[8];
+            for (int dt = 0; dt < NDT; ++dt) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[8 * s + e], f, -c));
-                    if (TAIL && !live(8 * s + e)) p[e] = 0.0f;
-                }
-                const uint32_t a0 = attn_pack_h2(p[0], p[1]), a1 = attn_pack_h2(p[2], p[3]);
-                const uint32_t b0 = attn_pack_h2(p[4], p[5]), b1 = attn_pack_h2(p[6], p[7]);
-                float ls = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2_a, a0), h2_one, 0.0f, false);
-                ls = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2_a, a1), h2_one, ls, false);
-                ls = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2_a, b0), h2_one, ls, false);
-                ls = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2_a, b1), h2_one, ls, false);
-                v4i_a pf;                                      // as they are (attn_vt_pos)
-                pf[0] = (int) a0; pf[1] = (int) a1; pf[2] = (int) b0; pf[3] = (int) b1;
-                pn[s] = __builtin_bit_cast(v8h_a, pf);
-                return ls;
-        };
-        auto weights = [&]() {
-            const float c = SAGE ? __builtin_fmaf(kScoreBias, f, m) : m;
-            float ls[4];
-#pragma unroll
-            for (int s = 0; s < 4; ++s) ls[s] = chunk(s, c);
-            return (ls[0] + ls[1]) + (ls[2] + ls[3]);
-        };
-        // First against the current reference m, with no max: a weight past half's range (a score more than about
-        // 16 above m, or m not yet set) rounds to infinity and makes the lane's sum infinite. Only then the tile's
-        // max: m moves when it passes m by more than 8 (as in attn_kernel), O and l are rescaled and the weights
-        // computed again (each at most 1 then). O / l does not depend on m.
-        float lt = weights();
-        if (__any(!(lt <= 3.0e38f))) {
-            asm volatile("" ::: "memory");
-            float mt[16];
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const float u = TAIL && !live(i) ? -INFINITY : x[i], w = TAIL && !live(i + 16) ? -INFINITY : x[i + 16];
-                mt[i] = fmaxf(u, w);
+                for (int gq = 0; gq < NG; ++gq)
+                    o[gq][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[s][dt], pb[gq][s], o[gq][dt], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                if (s == 0 && dt == 1) issue(prev);
+                if (SAGE && s == 0 && dt == 2) ks_next = ksc[(t0 + (t + 1 < T ? t + 1 : t)) / 2];
+                if (s == 1 && dt < KP) kread(next, dt);
+                __builtin_amdgcn_sched_barrier(0);
             }
-#pragma unroll
-            for (int w = 8; w >= 1; w /= 2)
-#pragma unroll
-                for (int i = 0; i < w; ++i) mt[i] = fmaxf(mt[i], mt[i + w]);
-            const float mx = (attn_pair_max(mt[0]) - (SAGE ? kScoreBias : 0.0f)) * f;
-            if (mx > m + 8.0f) {
-                const float mn = fmaxf(m, mx);
-                alpha = __builtin_amdgcn_exp2f(m - mn);
-                m = mn;
-                l = l * alpha;
-            }
-            lt = weights();
-        }
-        l = l + lt;
-    };
-    using yes = std::true_type;
-    using no = std::false_type;
-    const bool ragged = S % kAttnRows != 0 && t0 + T == Tall;   // this range ends with the sequence's cut tile
-    // Step t: refill the ring (tile t + NS - 1); the scores of tile t + 1 (DS); tile t's P v products (DPV) with the
-    // softmax of tile t + 1 (independent of them) between them; O's rescale, if the softmax moved the reference; the
-    // wait for tile t + 2 and one barrier. Tile j is read in steps j - 1 (K) and j (V^T); its stage is refilled at
-    // step j + 1, after the barrier that ends step j.
-    auto step = [&](int t, auto s_tag, auto pv_tag, auto tail_tag) {
-        constexpr bool DS = decltype(s_tag)::value, DPV = decltype(pv_tag)::value;
-        if (t >= 0) issue(t + NS - 1);
-        if constexpr (DS) scores(t);
-        if constexpr (DPV) pv(t);
-        float alpha = 1.0f;
-        if constexpr (DS) softmax(t, tail_tag, alpha);       // the compiler places it between the P v products
-        if constexpr (DPV) {
-            if (alpha != 1.0f) {
-#pragma unroll
-                for (int dt = 0; dt < NDT; ++dt) o[dt] = o[dt] * alpha;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) pb[u] = pn[u];
-        wait_vm<LATER>();                                      // tile t + 2 is in (the barrier publishes it)
-        lds_barrier();
+        prev = cur;
+        cur = next;
     };
 
-    // q's fragments and the scales are in before the first direct load: the compiler's own wait counts then see
-    // nothing in flight inside the loop (the direct loads are not counted by it)
+    // q's fragments are in before the first direct load: the compiler's own wait counts then see nothing in flight
+    // inside the loop (the direct loads are not counted by it)
     wait_vm<0>();
-    for (int t = 0; t < NS - 1; ++t) issue(t);
-    wait_vm<(NS - 2) * (KI + VI)>();
-    lds_barrier();                                             // tile 0 is in; qmax is written
-    if constexpr (SAGE) {
-        if (P.qraw) {
-            // q's codes (attn_qk_prep_vec_kernel's arithmetic): the 64-row block's max over both wavefronts
-            const float m = fmaxf(qm, qmax[wave ^ 1]);
-            const float inv = m > 0.0f ? 127.0f / m : 0.0f;
+    for (int t = 0; t < NS - 1; ++t) issue(t * STAGE);
+    wait_vm<(NS - 2) * L>();
+    lds_barrier();                                             // tile 0 is in
 #pragma unroll
-            for (int kk = 0; kk < NQF; ++kk) {
-                v4i_a w;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    uint32_t b = 0;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float cc = fminf(fmaxf(roundf(qx[kk * FR + 4 * i + e] * inv), -127.0f), 127.0f);
-                        b |= (uint32_t) ((int) cc & 255) << (8 * e);
-                    }
-                    w[i] = (int) b;
-                }
-                qf[kk] = w;
-            }
-            fq = m / 127.0f * P.c;
-        }
-    }
-    if (T == 1 && ragged) step(-1, yes{}, no{}, yes{});
-    else step(-1, yes{}, no{}, no{});
+    for (int u = 0; u < KP; ++u) kread(0, u);   // (KP <= NDT: a fragment behind each pair of products)
+    const int full = S % kAttnVT != 0 && t0 + T == Tall ? T - 1 : T;   // the tiles before the sequence's cut one
     int t = 0;
-    for (; t < T - 2; ++t) step(t, yes{}, yes{}, no{});
-    if (t == T - 2) {                                          // the scores of the last tile
-        if (ragged) step(t, yes{}, yes{}, yes{});
-        else step(t, yes{}, yes{}, no{});
-        ++t;
-    }
-    step(t, no{}, yes{}, no{});                                // step T - 1: the last P v products
+    for (; t < full; ++t) step(t, std::false_type{});
+    if (t < T) step(t, std::true_type{});
     wait_vm<0>();                                              // no direct load may land after the block ends
 
     // ---- a split block: O, m and l of its key range for attn_merge_kernel ----
     if (slot >= 0) {
-        const int64_t row = (int64_t) slot * kAttnPPQ + 32 * wave + ql;
-        float* po = P.po + row * DK;
 #pragma unroll
-        for (int dt = 0; dt < NDT; ++dt)
+        for (int gq = 0; gq < NG; ++gq) {
+            const int64_t row = (int64_t) slot * kAttnPPQ + 64 * wave + 32 * gq + ql;
+            float* po = P.po + row * DK;
 #pragma unroll
-            for (int gq = 0; gq < 4; ++gq)
-                *reinterpret_cast<float4*>(po + 32 * dt + 8 * gq + 4 * hl) =
-                    make_float4(o[dt][4 * gq], o[dt][4 * gq + 1], o[dt][4 * gq + 2], o[dt][4 * gq + 3]);
-        const float lsum = attn_pair_sum(l);                   // m is the same in both lanes of the query
-        if (hl == 0) *reinterpret_cast<float2*>(P.pml + 2 * row) = make_float2(m, lsum);
+            for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                for (int q4 = 0; q4 < 4; ++q4)
+                    *reinterpret_cast<float4*>(po + 32 * dt + 8 * q4 + 4 * hl) =
+                        make_float4(o[gq][dt][4 * q4], o[gq][dt][4 * q4 + 1], o[gq][dt][4 * q4 + 2], o[gq][dt][4 * q4 + 3]);
+            const float lsum = attn_pair_sum(l[gq]);           // m is the same in both lanes of the query
+            if (hl == 0) *reinterpret_cast<float2*>(P.pml + 2 * row) = make_float2(m[gq], lsum);
+        }
         return;
     }
 
     // ---- out = O / l, rounded to half, in out's type ----
-    // Through LDS, so that the stores are whole rows: each wavefront stages its 32 queries, 256 bytes of features a
-    // row per pass (all 128 features of a 16-bit out, 64 of a float32 one), into an area of its own in the ring
-    // (free once every wavefront is past its last P v products), then reads it back as 16-byte chunks, four rows an
-    // instruction.
-    const float inv = 1.0f / attn_pair_sum(l);
+    // Through LDS, so that the stores are whole rows: each wavefront stages 32 queries, 256 bytes of features a row per
+    // pass (all 128 features of a 16-bit out, 64 of a float32 one), into an area of its own in the ring (free once
+    // every wavefront is past its last P v products), then reads it back as 16-byte chunks, four rows an instruction.
     lds_barrier();
     constexpr int OPITCH = 256 + 16;                           // bytes a staged row (16 of pad: rows on other banks)
-    static_assert(8 * 32 * OPITCH <= NS * STAGE, "the output staging fits in the ring");
+    static_assert(4 * 32 * OPITCH <= NS * STAGE, "the output staging fits in the ring");
     int8_t* ost = lds + wave * 32 * OPITCH;
     auto store = [&](auto dt_tag) {
         constexpr int OUT = decltype(dt_tag)::value;
         constexpr int esz = OUT == H3S_F32 ? 4 : 2;
         constexpr int FP = 256 / esz, NPASS = DK / FP, DTP = FP / 32;   // features, passes, o[] registers a pass
 #pragma unroll
-        for (int pass = 0; pass < NPASS; ++pass) {
+        for (int gq = 0; gq < NG; ++gq) {
+            const float inv = 1.0f / attn_pair_sum(l[gq]);
 #pragma unroll
-            for (int d = 0; d < DTP; ++d)
+            for (int pass = 0; pass < NPASS; ++pass) {
 #pragma unroll
-                for (int gq = 0; gq < 4; ++gq) {
-                    // registers 4 gq .. 4 gq + 3 of o[dt]: features 32 dt + 8 gq + 4 hl + (0..3)
-                    const int dt = pass * DTP + d;
-                    float v[4];
+                for (int d = 0; d < DTP; ++d)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) v[i] = round_f16(o[dt][4 * gq + i] * inv);
-                    int8_t* at = ost + ql * OPITCH + (32 * d + 8 * gq + 4 * hl) * esz;
-                    if constexpr (OUT == H3S_F32) *reinterpret_cast<float4*>(at) = make_float4(v[0], v[1], v[2], v[3]);
-                    else if constexpr (OUT == H3S_BF16) *reinterpret_cast<uint2*>(at) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
-                    else *reinterpret_cast<uint2*>(at) = make_uint2(pack_f16(v[0], v[1]), pack_f16(v[2], v[3]));
+                    for (int q4 = 0; q4 < 4; ++q4) {
+                        // registers 4 q4 .. 4 q4 + 3 of o[dt]: features 32 dt + 8 q4 + 4 hl + (0..3)
+                        const int dt = pass * DTP + d;
+                        float v[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) v[i] = round_f16(o[gq][dt][4 * q4 + i] * inv);
+                        int8_t* at = ost + ql * OPITCH + (32 * d + 8 * q4 + 4 * hl) * esz;
+                        if constexpr (OUT == H3S_F32) *reinterpret_cast<float4*>(at) = make_float4(v[0], v[1], v[2], v[3]);
+                        else if constexpr (OUT == H3S_BF16) *reinterpret_cast<uint2*>(at) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+                        else *reinterpret_cast<uint2*>(at) = make_uint2(pack_f16(v[0], v[1]), pack_f16(v[2], v[3]));
+                    }
+                wave_lds_sync();
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const int ch = lane + 64 * k, r = ch / 16, c = ch % 16;
+                    const uint4 val = *reinterpret_cast<const uint4*>(ost + r * OPITCH + 16 * c);
+                    const int64_t qr = q0 + 32 * gq + r;
+                    if (qr < S) *reinterpret_cast<uint4*>(reinterpret_cast<char*>(P.out) + ((qr * P.H + h) * DK + pass * FP) * esz + 16 * c) = val;
                 }
-            wave_lds_sync();
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int ch = lane + 64 * k, r = ch / 16, c = ch % 16;
-                const uint4 val = *reinterpret_cast<const uint4*>(ost + r * OPITCH + 16 * c);
-                const int64_t qr = q0 + r;
-                if (qr < S) *reinterpret_cast<uint4*>(reinterpret_cast<char*>(P.out) + ((qr * P.H + h) * DK + pass * FP) * esz + 16 * c) = val;
+                wave_lds_sync();
             }
-            wave_lds_sync();
         }
     };
     if (P.out_dt == H3S_F32) store(std::integral_constant<int, H3S_F32>{});
@@ -1040,7 +1056,7 @@ __global__ __launch_bounds__(512, 1) void attn_pl_kernel(AttnArgs P) {
 }
 
 // The split blocks' results combined: per query, M = max m_s, O = sum 2^(m_s - M) O_s, l = sum 2^(m_s - M) l_s,
-// out = O / l rounded to half, in out's type (as the pipelined kernel's own epilogue). One thread a query and four
+// out = O / l rounded to half, in out's type (as the wide kernel's own epilogue). One thread a query and four
 // features of the DK = 128.
 __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs P, int64_t tail) {
     constexpr int DK = 128;

@@ -287,3 +287,30 @@ def test_attention_causal_head_sizes(dev, dt, L, Hq, Hkv, D):
     out = new(dev, DTS[dt], [L, Hq * D])
     ops.attention_causal(ops.Rows(qt, 0, qs, L, Hq, D), ops.Rows(kvt, 0, kvs, L, Hkv, D), ops.Rows(kvt, Hkv * D, kvs, L, Hkv, D), out)
     check(out.to_numpy().ravel(), want, dt, f"causal L={L} Hq={Hq} Hkv={Hkv} D={D}")
+
+
+@pytest.mark.parametrize("sage", [True, False])
+@pytest.mark.parametrize("S", [1, 31, 32, 33, 63, 64, 65, 96, 97, 127, 160, 192, 193, 224, 255, 256, 257, 300, 511, 513])
+def test_attention_wide_tiles(dev_sage, dev_16, sage, S):
+    """The wide kernel (heads of 128) around its 32-key tiles, the 64-row scale blocks, the rings of six and four stages
+    (sequences shorter and longer than they hold) and the 256-query blocks; the rows of q, k and v inside wider rows."""
+    H, D = 3, 128
+    stride = 3 * H * D
+    q, k, v = qkv(110 + S, S, H, D, o.BF16, stride)
+    want = o.attention(q, k, v, o.BF16, S, H, D, stride, out_dt=o.F32, sage=sage)
+    want = want[0] if sage else want
+    got = run(dev_sage if sage else dev_16, q, k, v, o.BF16, S, H, D, stride, o.F32)
+    check(got, want, o.F32, f"wide tiles S={S}")
+
+
+@pytest.mark.parametrize("sage", [True, False])
+@pytest.mark.parametrize("dt", [o.BF16, o.F16, o.F32])
+def test_attention_wide_split_ranges(dev_split, sage, dt):
+    """Split blocks whose key ranges end inside a scale block (47 tiles of 32 keys in ranges of 6): each part's scales,
+    masks and partial sums, for every type of q."""
+    S, H, D = 1500, 2, 128
+    q, k, v = qkv(131, S, H, D, dt, H * D)
+    want = o.attention(q, k, v, dt, S, H, D, H * D, out_dt=o.F32, sage=sage)
+    want = want[0] if sage else want
+    got = run(dev_split[(sage, "default")], q, k, v, dt, S, H, D, H * D, o.F32)
+    check(got, want, o.F32, f"wide split {sage}")
