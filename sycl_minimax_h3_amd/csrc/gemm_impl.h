@@ -553,8 +553,7 @@ __global__ __launch_bounds__(256) void gemm_merge_kernel(GemmArgs P) {
 // the round's share it removes, and the merge costs about 15 us: fc2's 1386 tiles at 16896 x 14336 -> 5376 took
 // 1191-1194 against 1211-1221 us (2 parts), 3864 at 47104 tokens 3258-3261 against 3322 us (8 parts); with 7168-byte
 // rows, 16896 tokens lost 1.5 % (622 against 608-618 us) and 47104 gained 1 %.
-// A launch of at most half as many tiles as CUs (a narrow product: a LoRA's first factor, 16896 x 5376 -> 64, is 66
-// tiles) splits every tile the same way, where that pays: there the split spreads one round's work over more CUs
+// A launch of at most half as many tiles as CUs (a narrow product: 16896 x 5376 -> 256 is 66 tiles) splits every tile the same way, where that pays: there the split spreads one round's work over more CUs
 // instead of shortening a last round. A tile takes about 1.2 us a K step and a merge about 3 us plus 0.05 us a part
 // (its 256 KiB written and read), so the split is taken when 1.2 nk (1 - 1/s) > 0.05 T s + 3 (T tiles, s parts).
 inline void gemm_plan_split(int64_t tiles, int64_t nk, int cus, int* main_tiles, int* split) {

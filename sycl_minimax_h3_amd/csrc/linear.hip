@@ -1,13 +1,13 @@
 // linear.hip - the plain (float) linear layers of kernels/h3sycl.h:87-93: h3s_linear (out = x w^T + bias),
 // h3s_linear_acc (out += x w^T + bias, a LoRA's second factor) and h3s_scale_rows (kernels/h3sycl.cpp:656-739).
 // bfloat16 and half operands with K a multiple of 32 run on the matrix cores in gemm_impl.h's pipeline
-// (gemm_f16_kernel): float32 accumulation, and the epilogue adds the bias (and the old output) in float32 and rounds
+// (gemm_f16_kernel), or gemm_skinny.h's where one side has few rows (not h3s_linear_acc): float32 accumulation, and the epilogue adds the bias (and the old output) in float32 and rounds
 // once to the output type, as the reference's matmul post-ops do, with no intermediate in memory. Every other call
 // (float32 operands, other K, unaligned rows) runs on rocBLAS (a plain library GEMM, float32 accumulation, on the
 // context's stream) into a float32 scratch, a chunk of rows at a time, and the same epilogue as a kernel of its own.
 #include <rocblas/rocblas.h>
 
-#include "gemm_impl.h"
+#include "gemm_skinny.h"
 
 namespace h3 {
 
@@ -130,12 +130,77 @@ static int linear_mfma(Ctx* c, const char* fn, const void* x, int dt, int64_t M,
     return launched(fn);
 }
 
+template <int OP, int MT, int NT, bool SWAP>
+static void skinny_one(Ctx* c, const SkinnyArgs& P) {
+    const int64_t tiles = (int64_t) P.ts * P.tl;
+    gemm_skinny_kernel<OP, MT, NT, SWAP><<<(unsigned) (tiles * P.parts), kSkinnyThreads, 0, c->stream>>>(P);
+    if (P.parts > 1) skinny_merge_kernel<MT, NT, SWAP><<<(unsigned) (tiles * (64 * MT * 64 * NT / 4 / 256)), 256, 0, c->stream>>>(P);
+}
+template <int OP, bool SWAP>
+static void skinny_mt(Ctx* c, const SkinnyArgs& P, int mt, int nt) {
+#define H3_SK(MM) case MM: if (nt == 2) skinny_one<OP, MM, 2, SWAP>(c, P); else skinny_one<OP, MM, 1, SWAP>(c, P); break;
+    switch (mt) {
+        H3_SK(1) H3_SK(2) H3_SK(3) H3_SK(4)
+    }
+#undef H3_SK
+}
+// The tile (64 mt rows of S, 64 nt of L) and the parts along K of an S x L product of nk K steps, by the least estimated
+// time in microseconds (measured over S = 16 .. 512 rows against the DiT's layers and L = 300 .. 47104 rows against 16 ..
+// 128, the choice is within 10 % of the fastest of all tiles and parts): a CU takes about 2.4 ns a row and step and at
+// least 250 ns a step, the blocks run in rounds of one a CU, memory gives about 5 TB/s (7 for what the 256 MB cache beside
+// it may hold), and parts cost their float32 sums written and read once and the merge's launch.
+struct SkinnyPlan { int mt, nt, parts; double us; };
+static SkinnyPlan skinny_plan(int64_t S, int64_t L, int64_t nk, int cus) {
+    SkinnyPlan best{0, 0, 0, 1e300};
+    const int64_t ts = (S + 255) / 256;
+    const int mt = (int) ((S + 64 * ts - 1) / (64 * ts));
+    const int64_t rows = (S + ts - 1) / ts;
+    for (int nt = 1; nt <= 2; ++nt)
+        for (int parts = 1; parts <= 8; ++parts) {
+            if (parts > 1 && 4 * parts > nk) break;              // at least 4 steps a part
+            const int64_t blocks = ts * ((L + 64 * nt - 1) / (64 * nt)) * parts;
+            const double run = (double) ((blocks + cus - 1) / cus) * (double) ((nk + parts - 1) / parts) *
+                               std::max(0.25, 0.0024 * (double) (rows + 64 * nt));
+            const double bytes = (double) (S + L) * (double) nk * kGemmBK, floor = bytes / (bytes > 256e6 ? 5e6 : 7e6);
+            const double us = std::max(run, floor) + (parts > 1 ? 2.0 + (double) parts * (double) S * (double) L * 8 / 3.5e6 : 0.0);
+            if (us < best.us) best = {mt, nt, parts, us};
+        }
+    return best;
+}
+// h3s_linear with few rows on one side (gemm_skinny.h): at most 512 rows of x, or at most 128 of w. Above, gemm_impl.h's
+// tiles have the rows to fill them (768 rows 5376 -> 5376: 65 against 66 us at the best tile here; 256 rows of w at 16896
+// tokens 95 against 137). 1: not a shape it takes.
+static int linear_skinny(Ctx* c, const char* fn, const void* x, int dt, int64_t M, int64_t K, const void* w, int64_t N,
+                         const float* bias, void* out, int out_dt) {
+    const int64_t kb = 2 * K, nk = (kb + kGemmBK - 1) / kGemmBK;
+    SkinnyPlan p{0, 0, 0, 1e300};
+    bool swap = false;
+    if (M <= 512) p = skinny_plan(M, N, nk, c->cus);
+    if (N <= 128) {
+        const SkinnyPlan q = skinny_plan(N, M, nk, c->cus);
+        if (q.us < p.us) { p = q; swap = true; }
+    }
+    if (!p.mt) return 1;
+    const int64_t S = swap ? N : M, L = swap ? M : N;
+    const int64_t ts = (S + 64 * p.mt - 1) / (64 * p.mt), tl = (L + 64 * p.nt - 1) / (64 * p.nt);
+    if (ts * tl * 64 > 0x7fffffff) return 1;                     // (blocks, and the merge's, within 32 bits)
+    SkinnyArgs P{(const int8_t*) (swap ? w : x), (const int8_t*) (swap ? x : w), S, L, kb, bias, out, out_dt, (int) ts, (int) tl, p.parts, nullptr};
+    // (no room for the partial sums under the memory cap: each tile whole)
+    if (P.parts > 1 && !(P.part = c->scratch<float>(Ctx::GEMM_PART, (size_t) (ts * tl * P.parts) * (64 * p.mt * 64 * p.nt)))) P.parts = 1;
+    if (dt == H3S_BF16) { if (swap) skinny_mt<GEMM_BF16, true>(c, P, p.mt, p.nt); else skinny_mt<GEMM_BF16, false>(c, P, p.mt, p.nt); }
+    else { if (swap) skinny_mt<GEMM_F16, true>(c, P, p.mt, p.nt); else skinny_mt<GEMM_F16, false>(c, P, p.mt, p.nt); }
+    return launched(fn);
+}
+
 // the product x [M, K] . w^T (w [N, K]), both in dt, into out (or out +=): on the matrix cores, or on rocBLAS a
 // chunk of rows at a time
 static int linear(Ctx* c, const char* fn, const void* x, int dt, int64_t M, int64_t K, const void* w, int64_t N,
                   const float* bias, void* out, int out_dt, bool acc) {
     if (K > 0x7fffffff || N > 0x7fffffff) return fail(std::string(fn) + ": K and N must be below 2^31");
-    if (mfma_takes(dt, x, w, out, M, K, N)) return linear_mfma(c, fn, x, dt, M, K, w, N, bias, out, out_dt, acc);
+    if (mfma_takes(dt, x, w, out, M, K, N)) {
+        const int r = acc ? 1 : linear_skinny(c, fn, x, dt, M, K, w, N, bias, out, out_dt);
+        return r != 1 ? r : linear_mfma(c, fn, x, dt, M, K, w, N, bias, out, out_dt, acc);
+    }
     rocblas_handle h = blas_of(c);
     if (!h) return -1;
     // rows a chunk: the float32 product of a chunk takes at most 256 MiB (and at most 8192 rows, as the reference)

@@ -3,7 +3,7 @@ products: h3s_linear, h3s_linear_acc (row chunks included) and h3s_scale_rows. T
 whose accumulation order is not restated: the parity tolerance (relative L2 < 1e-3, one ulp of the output type).
 bfloat16 and half operands with K a multiple of 32 run on the matrix-core kernel (256 x 256 tiles: partial tiles at
 every edge, K steps of 64 elements with a last half step where K is an odd multiple of 32, the long-K tile order
-from K = 6144; launches of few tiles split along K: 2000 x 1024 -> 64 or 100, 8 tiles in 8 parts each); K = 200 and
+from K = 6144); h3s_linear with at most 512 rows of x or 128 of w on the few-rows kernel; K = 200 and
 float32 operands run on rocBLAS with the separate epilogue."""
 import numpy as np
 import pytest
@@ -45,6 +45,16 @@ def test_linear(dev, dt, out_dt, M, K, N, bias):
     layer = ops.Linear(up(dev, w, DTS[dt], [N, K]), up(dev, b, "F32", [N]) if bias else None)
     layer.forward(up(dev, x, DTS[dt], [M, K]), out)
     close(out.to_numpy(), want, out_dt, "linear")
+
+
+# gemm_skinny.h's tiles and parts (at most 512 rows of x, or at most 128 of w): one row on either side, the edges of the
+# 64-row tiles along S and L, S past 256 rows (two tiles), a single K step, last half steps in one part and in several
+@pytest.mark.parametrize("M,K,N", [(1, 32, 8), (1, 4096, 1), (64, 64, 64), (65, 992, 129), (128, 1056, 333), (192, 2048, 66), (193, 544, 1000),
+                                   (256, 4128, 128), (257, 2080, 130), (512, 480, 4100), (511, 8192, 72), (513, 480, 128), (1030, 7168, 30),
+                                   (20000, 96, 65), (700, 4128, 127)])
+@pytest.mark.parametrize("dt,out_dt,bias", [(o.BF16, o.BF16, True), (o.F16, o.F16, False), (o.BF16, o.F32, True)])
+def test_linear_few_rows(dev, dt, out_dt, bias, M, K, N):
+    test_linear(dev, dt, out_dt, M, K, N, bias)
 
 
 @pytest.mark.parametrize("M,K,N", [(8300, 128, 64), (700, 1024, 600), (300, 96, 260), (130, 200, 70)])
