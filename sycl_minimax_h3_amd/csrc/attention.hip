@@ -12,7 +12,7 @@ namespace h3 {
 
 // q of Hq heads (row stride qs) and k, v of Hkv heads (row stride kvs) prepared into aq [Hq, Sp, DK], ak [Hkv, Sp, DK]
 // (int8 codes with their scales for SAGE, else half) and av [Hkv, DK, Sp] (half), DK = attn_dk(D), zero past D
-// (q_in_kernel: the wide kernel forms q's fragments from q itself, so q is not prepared)
+// (q_in_kernel: the attention kernel forms q's fragments from q itself, so q is not prepared)
 template <int DT>
 static void prep(Ctx* c, const void* q, const void* k, const void* v, int64_t S, int64_t Sp, int64_t Hq, int64_t Hkv, int D,
                  int64_t qs_stride, int64_t kv_stride, bool sage, bool q_in_kernel, int8_t* aq, int8_t* ak, uint16_t* av,
@@ -39,6 +39,23 @@ static void prep(Ctx* c, const void* q, const void* k, const void* v, int64_t S,
         }
 #undef H3_QK
     };
+    // k and v: together where both take the 16-byte form
+    auto kv = [&](const float* mean, float* sc) {
+#define H3_KV(SG, DD) attn_kv_prep_vec_kernel<DT, SG, DD><<<2 * kvblocks, 256, 0, c->stream>>>(k, v, S, Sp, kv_stride, mean, ak, sc, av)
+        if (!vec) {
+            qk(k, kv_stride, kvblocks, mean, ak, sc);
+            attn_v_prep_kernel<DT><<<kvblocks, 256, 0, c->stream>>>(v, S, Sp, D, DK, kv_stride, av);
+        } else if (sage) {
+            if (D == 256) H3_KV(true, 256);
+            else if (D == 128) H3_KV(true, 128);
+            else H3_KV(true, 64);
+        } else {
+            if (D == 256) H3_KV(false, 256);
+            else if (D == 128) H3_KV(false, 128);
+            else H3_KV(false, 64);
+        }
+#undef H3_KV
+    };
     if (sage) {
         // k's mean per (head, feature) of the D features; the 16-byte form takes 16 features a block, or 32 where 16
         // would make more blocks than the device runs at once
@@ -47,18 +64,16 @@ static void prep(Ctx* c, const void* q, const void* k, const void* v, int64_t S,
         if (vec && wide) attn_kmean_kernel<DT, kKmeanFeatWide><<<(unsigned) (hd / kKmeanFeatWide), 256, 0, c->stream>>>(k, S, kv_stride, km);
         else if (vec && hd % kKmeanFeat == 0) attn_kmean_kernel<DT, kKmeanFeat><<<(unsigned) (hd / kKmeanFeat), 256, 0, c->stream>>>(k, S, kv_stride, km);
         else attn_kmean_rows_kernel<DT><<<(unsigned) ((hd + 255) / 256), 256, 0, c->stream>>>(k, S, hd, kv_stride, km);
-        if (!q_in_kernel) qk(q, qs_stride, qblocks, nullptr, aq, qs);
-        qk(k, kv_stride, kvblocks, km, ak, ks);
-    } else {
-        if (!q_in_kernel) qk(q, qs_stride, qblocks, nullptr, aq, nullptr);
-        qk(k, kv_stride, kvblocks, nullptr, ak, nullptr);
     }
-    if (!vec) attn_v_prep_kernel<DT><<<kvblocks, 256, 0, c->stream>>>(v, S, Sp, D, DK, kv_stride, av);
-    else if (D == 256) attn_v_prep_vec_kernel<DT, 256><<<kvblocks, 256, 0, c->stream>>>(v, S, Sp, kv_stride, av);
-    else if (D == 128) attn_v_prep_vec_kernel<DT, 128><<<kvblocks, 256, 0, c->stream>>>(v, S, Sp, kv_stride, av);
-    else attn_v_prep_vec_kernel<DT, 64><<<kvblocks, 256, 0, c->stream>>>(v, S, Sp, kv_stride, av);
+    if (!q_in_kernel) qk(q, qs_stride, qblocks, nullptr, aq, sage ? qs : nullptr);
+    kv(sage ? km : nullptr, sage ? ks : nullptr);
 }
 
+// Whether the causal form takes two key groups a block: where the launch's time is the walk of its longest blocks (few heads,
+// long rows). bfloat16, heads of 128: 8 heads 2048 tokens 48.9 -> 40.9 us, 32 heads 600 tokens 22.1 -> 20.5, 2048 tokens
+// 61.7 -> 57.7; but 64 heads 600 tokens 23.7 -> 24.7, 2048 tokens 94.5 -> 103 (the blocks fill the device: there two blocks of
+// one group a CU run without a common barrier), and 100 tokens 11.3 -> 12.4 (two tiles: nothing to share out)
+static bool attn_causal_groups(int64_t L, int64_t Hq, int cus) { return L >= 512 && 8 * Hq <= cus; }
 // one sequence: S query rows of Hq heads (row stride qs_stride) over S key/value rows of Hkv heads (kv_stride);
 // causal: query i sees keys 0 .. i (the 16-bit form, as the reference's causal kernel computes in float)
 static int attention_one(Ctx* c, const char* fn, const void* q, const void* k, const void* v, int dt, int64_t S, int64_t Hq,
@@ -72,8 +87,14 @@ static int attention_one(Ctx* c, const char* fn, const void* q, const void* k, c
     const int64_t Sp = (S + qblock - 1) / qblock * qblock, nbp = Sp / kAttnRows;
     const int64_t esz = sage ? 1 : 2, DK = attn_dk(D);
     if (Hq * (Sp / qblock) > 0x7fffffff) return fail(std::string(fn) + ": too many query blocks");
-    // the wide kernel reads q's rows itself where they are whole 16-byte vectors (no prepared q then)
-    const bool q_in_kernel = pp && aligned16(q) && (qs_stride * elem_size(dt)) % 16 == 0;
+    // the wide kernel, and the 16-bit form of the others, read q's rows themselves where they are whole 16-byte vectors of
+    // unpadded heads (no prepared q then: one launch less, and q neither written nor read again)
+    // (a block of the others then writes out while another may still read q: an out that overlaps q otherwise than row on
+    // row has q prepared first)
+    const char *qb0 = (const char*) q, *ob0 = (const char*) out;
+    const bool apart = ob0 + S * Hq * D * elem_size(out_dt) <= qb0 || qb0 + S * qs_stride * elem_size(dt) <= ob0 ||
+                       (ob0 == qb0 && qs_stride == Hq * D && elem_size(dt) == elem_size(out_dt));
+    const bool q_in_kernel = (pp || (!sage && apart)) && D == DK && aligned16(q) && (qs_stride * elem_size(dt)) % 16 == 0;
     int8_t* aq = q_in_kernel ? nullptr : c->scratch<int8_t>(Ctx::ATT_Q, (size_t) (Sp * Hq * DK * esz));
     const size_t over = pp ? kAttnOver : 0;                   // what its last direct loads read past the end
     int8_t* ak = c->scratch<int8_t>(Ctx::ATT_K, (size_t) (Sp * Hkv * DK * esz) + over);
@@ -137,6 +158,9 @@ static int attention_one(Ctx* c, const char* fn, const void* q, const void* k, c
         if (sage) attn_pl_kernel<true, 6><<<grid, 256, 0, c->stream>>>(P);
         else attn_pl_kernel<false, 4><<<grid, 256, 0, c->stream>>>(P);
         if (tail) attn_merge_kernel<<<(unsigned) ((tail * kAttnPPQ * 32 + 255) / 256), 256, 0, c->stream>>>(P, tail);
+    } else if (causal && DK <= 128 && attn_causal_groups(S, Hq, c->cus)) {
+        if (DK == 128) { if (pad) attn_kernel<false, 128, true, true, 2><<<grid, 512, 0, c->stream>>>(P); else attn_kernel<false, 128, true, false, 2><<<grid, 512, 0, c->stream>>>(P); }
+        else { if (pad) attn_kernel<false, 64, true, true, 2><<<grid, 512, 0, c->stream>>>(P); else attn_kernel<false, 64, true, false, 2><<<grid, 512, 0, c->stream>>>(P); }
     } else if (causal) H3_ATTN(false, true)
     else if (sage) {
         // (the int8 form only at 64 or 128 features, above)

@@ -257,21 +257,20 @@ __global__ __launch_bounds__(256) void attn_qk_prep_kernel(const void* __restric
     }
 }
 
-// The same two preparations with 16-byte loads, for rows that are 16-byte aligned (the tensor and the stride): a
 // Where key t of a 64-key tile sits in its row of v^T: inside each group of 16 keys the middle two quads swap
 // (bits 2 and 3 of t). The score products leave key 16 s + 8 (j / 4) + 4 hl + j % 4 of a query in register 8 s + j
 // of lane half hl; the P v product's second operand takes 8 consecutive k-indices per lane half from the registers
 // as they are, so its first operand (a 16-byte chunk of a v^T row) must hold those same 8 keys, in that order.
 __host__ __device__ constexpr int attn_vt_pos(int t) { return (t & ~12) | ((t & 4) << 1) | ((t & 8) >> 1); }
 
+// attn_qk_prep_kernel's work with 16-byte loads, for rows that are 16-byte aligned (the tensor and the stride): a
 // thread holds its chunks (V values each) of the block's 64 rows in registers between the max and the codes.
 template <int DT, bool SAGE, int D>
-__global__ __launch_bounds__(256) void attn_qk_prep_vec_kernel(const void* __restrict__ src, int64_t S, int64_t Sp,
-                                                               int64_t stride, const float* __restrict__ mean,
-                                                               int8_t* __restrict__ dst, float* __restrict__ scales) {
+__device__ __forceinline__ void attn_qk_prep_body(int block, const void* __restrict__ src, int64_t S, int64_t Sp, int64_t stride,
+                                                  const float* __restrict__ mean, int8_t* __restrict__ dst, float* __restrict__ scales) {
     constexpr int V = Vec<DT>::V, CPR = D / V, N = kAttnRows * CPR / 256;   // chunks a row, chunks a thread
     __shared__ float red[4];
-    const int64_t nbp = Sp / kAttnRows, b = blockIdx.x % nbp, h = blockIdx.x / nbp, r0 = b * kAttnRows;
+    const int64_t nbp = Sp / kAttnRows, b = block % nbp, h = block / nbp, r0 = b * kAttnRows;
     const int tid = threadIdx.x;
     const char* base = reinterpret_cast<const char*>(src) + (r0 * stride + h * D) * (int64_t) (16 / V);
     // k's mean at this thread's chunks, loaded before the rows so that both are in flight together (loaded after
@@ -350,14 +349,14 @@ __global__ __launch_bounds__(256) void attn_qk_prep_vec_kernel(const void* __res
 }
 
 template <int DT, int D>
-__global__ __launch_bounds__(256) void attn_v_prep_vec_kernel(const void* __restrict__ v, int64_t S, int64_t Sp,
-                                                              int64_t stride, uint16_t* __restrict__ vt) {
+__device__ __forceinline__ void attn_v_prep_body(int block, const void* __restrict__ v, int64_t S, int64_t Sp, int64_t stride,
+                                                 uint16_t* __restrict__ vt) {
     // PITCH: an odd number of 4-byte words a feature row (35), so the 16 chunks a wavefront's lanes write for one
     // token group fall in distinct banks (a pitch of 36 words put 8 lanes on each bank: 29.9 -> 21.4 us on average
     // over the attention calls of a benchmark run); the rows are then 4-byte aligned, read 4 bytes at a time
     constexpr int V = Vec<DT>::V, CPR = D / V, N = kAttnRows * CPR / 256, PITCH = kAttnRows + 6;
     __shared__ __attribute__((aligned(16))) uint16_t tile[D * PITCH];   // [feature][token], half bits
-    const int64_t nbp = Sp / kAttnRows, b = blockIdx.x % nbp, h = blockIdx.x / nbp, t0 = b * kAttnRows;
+    const int64_t nbp = Sp / kAttnRows, b = block % nbp, h = block / nbp, t0 = b * kAttnRows;
     const int tid = threadIdx.x;
     const char* base = reinterpret_cast<const char*>(v) + (t0 * stride + h * D) * (int64_t) (16 / V);
 #pragma unroll
@@ -379,6 +378,23 @@ __global__ __launch_bounds__(256) void attn_v_prep_vec_kernel(const void* __rest
         const uint32_t* row = reinterpret_cast<const uint32_t*>(tile + d * PITCH + t);
         *reinterpret_cast<uint4*>(vt + (h * Sp + t0) * D + 8 * u) = make_uint4(row[0], row[1], row[4], row[5]);
     }
+}
+
+template <int DT, bool SAGE, int D>
+__global__ __launch_bounds__(256) void attn_qk_prep_vec_kernel(const void* __restrict__ src, int64_t S, int64_t Sp,
+                                                               int64_t stride, const float* __restrict__ mean,
+                                                               int8_t* __restrict__ dst, float* __restrict__ scales) {
+    attn_qk_prep_body<DT, SAGE, D>((int) blockIdx.x, src, S, Sp, stride, mean, dst, scales);
+}
+// k (blocks [0, n)) and v (blocks [n, 2 n)) of the key/value heads in one launch
+template <int DT, bool SAGE, int D>
+__global__ __launch_bounds__(256) void attn_kv_prep_vec_kernel(const void* __restrict__ k, const void* __restrict__ v, int64_t S,
+                                                               int64_t Sp, int64_t stride, const float* __restrict__ mean,
+                                                               int8_t* __restrict__ kd, float* __restrict__ scales,
+                                                               uint16_t* __restrict__ vt) {
+    const int n = (int) (gridDim.x / 2), b = (int) blockIdx.x;
+    if (b < n) attn_qk_prep_body<DT, SAGE, D>(b, k, S, Sp, stride, mean, kd, scales);
+    else attn_v_prep_body<DT, D>(b - n, v, S, Sp, stride, vt);
 }
 
 // v of one head and 64 tokens to half, transposed: vt [H, DK, Sp]; tokens past S and features past D become zeros
@@ -432,8 +448,9 @@ struct AttnArgs {
     int nsplit, ts;
     float* po;                // [tail * nsplit, 256, DK] O before the division by l
     float* pml;               // [tail * nsplit, 256, 2] m and l
-    // the wide kernel with qraw set reads q from the caller's rows (stride qstride elements of type q_dt, 16-byte
-    // aligned) and forms its fragments itself, as attn_qk_prep_vec_kernel would (q and qs are then unused)
+    // with qraw set the wide kernel, and the 16-bit form of the others, read q from the caller's rows (stride qstride
+    // elements of type q_dt, 16-byte aligned, D = DK) and form its fragments themselves, as attn_qk_prep_vec_kernel would
+    // (q and qs are then unused)
     const void* qraw;
     int64_t qstride;
     int q_dt;
@@ -458,14 +475,34 @@ __device__ __forceinline__ float attn_pair_sum(float x) {
 
 // PAD: heads of D < DK features, or rows of out not on 16-byte boundaries: the output stores only features below D,
 // four at a time where they stay aligned
-template <bool SAGE, int DK, bool CAUSAL = false, bool PAD = false>
-__global__ __launch_bounds__(256, DK == 256 ? 1 : 3) void attn_kernel(AttnArgs P) {
+// KS 2: two groups of four wavefronts, each with a ring of its own, take every other key tile of the block's 128 queries
+// and meet at the end (group 1's O, m and l to group 0 through LDS): half the steps in a row, where a launch's time is its
+// longest block's walk.
+template <bool SAGE, int DK, bool CAUSAL = false, bool PAD = false, int KS = 1>
+__global__ __launch_bounds__(256 * KS, KS == 2 ? 2 : DK == 256 ? 1 : 3) void attn_kernel(AttnArgs P) {
     constexpr int ESZ = SAGE ? 1 : 2, RB = DK * ESZ, CPR = RB / 16, NQF = RB / 32;
     constexpr int KTB = kAttnRows * RB, VTB = DK * kAttnRows * 2, STAGE = KTB + VTB;
     constexpr int NDT = DK / 32;                               // 32-row tiles of V^T (32 features each)
-    __shared__ __attribute__((aligned(16))) int8_t lds[2 * STAGE];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, hl = lane >> 5, ql = lane & 31;
-    const int64_t h = blockIdx.x / P.nqb, qb = blockIdx.x % P.nqb, Sp = P.Sp, S = P.S;
+    static_assert(KS == 1 || (KS == 2 && !SAGE && DK <= 128 && KS * 2 * STAGE >= (NDT * 16 + 2) * 1024), "attn_kernel: key groups");
+    __shared__ __attribute__((aligned(16))) int8_t lds[KS * 2 * STAGE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) & 3, hl = lane >> 5, ql = lane & 31;
+    const int kg = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+    int64_t h = blockIdx.x / P.nqb, qb = blockIdx.x % P.nqb;
+    if constexpr (CAUSAL) {
+        // the blocks with the most keys first (in the order of the rows the longest started last: 2048 tokens x 64 heads,
+        // with q read here and k and v prepared in one launch, 150 -> 95 us, 300 tokens 24.1 -> 15.3); each XCD (blocks
+        // b % 8) a run of heads, which share k and v
+        const int b = (int) blockIdx.x, H = (int) P.H;
+        if (H % 8 == 0) {
+            const int hx = H / 8;
+            h = (b % 8) * hx + b / 8 % hx;
+            qb = P.nqb - 1 - b / 8 / hx;
+        } else {
+            h = b % H;
+            qb = P.nqb - 1 - b / H;
+        }
+    }
+    const int64_t Sp = P.Sp, S = P.S;
     const int64_t q0 = qb * kAttnQBlock + 32 * wave;          // this wavefront's first query
     const int64_t nbp = Sp / kAttnRows;
     // CAUSAL: query i sees keys 0 .. i, so the block stops at its last query
@@ -474,7 +511,35 @@ __global__ __launch_bounds__(256, DK == 256 ? 1 : 3) void attn_kernel(AttnArgs P
 
     // this lane's query fragments (second operand of the score products), held for the whole key walk
     v4i_a qf[NQF];
-    {
+    if (!SAGE && P.qraw) {
+        // from the caller's rows (D = DK, 16-byte aligned): the halves attn_qk_prep_vec_kernel would have written
+        auto qload = [&](auto dt_tag) {
+            constexpr int QDT = decltype(dt_tag)::value, qes = QDT == H3S_F32 ? 4 : 2, QV = 16 / qes;
+            const int64_t qi = q0 + ql;
+            const char* qrow = reinterpret_cast<const char*>(P.qraw) + ((qi < S ? qi : S - 1) * P.qstride + h * DK + 8 * hl) * qes;
+            uint4 raw[NQF][8 / QV];
+#pragma unroll
+            for (int kk = 0; kk < NQF; ++kk)
+#pragma unroll
+                for (int u = 0; u < 8 / QV; ++u) raw[kk][u] = *reinterpret_cast<const uint4*>(qrow + (16 * kk + QV * u) * qes);
+#pragma unroll
+            for (int kk = 0; kk < NQF; ++kk) {
+                float x[8];
+#pragma unroll
+                for (int u = 0; u < 8 / QV; ++u) {
+                    float y[QV];
+                    Vec<QDT>::unpack(raw[kk][u], y);
+#pragma unroll
+                    for (int e = 0; e < QV; ++e) x[QV * u + e] = qi < S ? y[e] : 0.0f;
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) qf[kk][e] = (int) pack_f16(x[2 * e], x[2 * e + 1]);
+            }
+        };
+        if (P.q_dt == H3S_BF16) qload(std::integral_constant<int, H3S_BF16>{});
+        else if (P.q_dt == H3S_F16) qload(std::integral_constant<int, H3S_F16>{});
+        else qload(std::integral_constant<int, H3S_F32>{});
+    } else {
         const int8_t* qrow = P.q + ((h * Sp + q0 + ql) * DK) * ESZ;
 #pragma unroll
         for (int kk = 0; kk < NQF; ++kk) qf[kk] = *reinterpret_cast<const v4i_a*>(qrow + 32 * kk + 16 * hl);
@@ -486,7 +551,7 @@ __global__ __launch_bounds__(256, DK == 256 ? 1 : 3) void attn_kernel(AttnArgs P
     const int8_t* kbase = P.k + g * Spk * RB;
     const uint16_t* vbase = P.vt + g * DK * Spk;
     auto issue = [&](int t, int st) {
-        int8_t* s = lds + st * STAGE;
+        int8_t* s = lds + (2 * kg + st) * STAGE;
         constexpr int KI = CPR / 4;                            // K instructions a wavefront
 #pragma unroll
         for (int j = 0; j < KI; ++j) {
@@ -514,13 +579,14 @@ __global__ __launch_bounds__(256, DK == 256 ? 1 : 3) void attn_kernel(AttnArgs P
     // one 64-key tile; TAIL: the last tile, which holds keys past S
     auto step = [&](int t, auto tail_tag) {
         constexpr bool TAIL = decltype(tail_tag)::value;
-        wait_vm<0>();
-        __syncthreads();                                       // tile t is in; every wavefront is done with tile t - 1
         // SAGE: the next tile's k scale, loaded before the tile's direct loads and waited for with them at the next
         // step (loaded after them, its wait here would wait for the whole tile)
         const float ks_next = SAGE ? P.ks[g * nbp + (t + 1 < ntiles ? t + 1 : t)] : 0.0f;
-        if (t + 1 < ntiles) issue(t + 1, (t + 1) & 1);
-        const int8_t* st = lds + (t & 1) * STAGE;
+        const int it = KS == 1 ? t : t / KS;                   // the group's step
+        if (t + KS < ntiles) issue(t + KS, (it + 1) & 1);
+        // (KS: a tile past this wavefront's last query has no live score)
+        if (KS > 1 && TAIL && (int64_t) t * kAttnRows > q0 + 31) return;
+        const int8_t* st = lds + (2 * kg + (it & 1)) * STAGE;
 
         // ---- scores: two 32-key halves of the tile ----
         float x[32];
@@ -571,7 +637,8 @@ __global__ __launch_bounds__(256, DK == 256 ? 1 : 3) void attn_kernel(AttnArgs P
         if (__any(mx > m + 8.0f)) {
             asm volatile("" ::: "memory");
             const float mn = fmaxf(m, mx);
-            const float alpha = __builtin_amdgcn_exp2f(m - mn);
+            // (KS: a lane may have seen no live score yet, m = mn = -infinity)
+            const float alpha = KS > 1 && m == mn ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
             m = mn;
             l = l * alpha;
 #pragma unroll
@@ -616,12 +683,47 @@ __global__ __launch_bounds__(256, DK == 256 ? 1 : 3) void attn_kernel(AttnArgs P
         l = l + ls;
         ks_cur = ks_next;
     };
-    issue(0, 0);
+    if (kg < ntiles) issue(kg, 0);
     // tiles with no key past S (and, CAUSAL, none past the block's first query) need no mask
     int full = (int) (S / kAttnRows);
     if constexpr (CAUSAL) full = full < (int) (qb * kAttnQBlock / kAttnRows) ? full : (int) (qb * kAttnQBlock / kAttnRows);
-    for (int t = 0; t < full; ++t) step(t, std::false_type{});
-    for (int t = full; t < ntiles; ++t) step(t, std::true_type{});
+    // before a step: its tile is in, and every wavefront is done with the tile before
+    auto ready = [&]() {
+        wait_vm<0>();
+        __syncthreads();
+    };
+    if constexpr (KS == 1) {
+        for (int t = 0; t < full; ++t) { ready(); step(t, std::false_type{}); }
+        for (int t = full; t < ntiles; ++t) { ready(); step(t, std::true_type{}); }
+    } else {
+        // (both groups take every barrier, the second one also where it has no last tile)
+        int t0 = 0;
+        for (; t0 + KS <= full; t0 += KS) { ready(); step(t0 + kg, std::false_type{}); }
+        for (; t0 < ntiles; t0 += KS) {
+            ready();
+            if (t0 + kg < ntiles) step(t0 + kg, std::true_type{});
+        }
+        __syncthreads();                                       // the stages are done with: LDS is the groups' now
+        float* ex = reinterpret_cast<float*>(lds) + wave * ((NDT * 16 + 2) * 64) + lane;
+        if (kg == 1) {
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) ex[(dt * 16 + i) * 64] = o[dt][i];
+            ex[NDT * 16 * 64] = m;
+            ex[(NDT * 16 + 1) * 64] = l;
+        }
+        __syncthreads();
+        if (kg == 1) return;
+        // (group 0 has seen key 0: its m is a number, or NaN as the scores are)
+        const float m1 = ex[NDT * 16 * 64], mn = fmaxf(m, m1);
+        const float a0 = __builtin_amdgcn_exp2f(m - mn), a1 = __builtin_amdgcn_exp2f(m1 - mn);
+        l = l * a0 + ex[(NDT * 16 + 1) * 64] * a1;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[dt][i] = o[dt][i] * a0 + ex[(dt * 16 + i) * 64] * a1;
+    }
 
     // ---- out = O / l, rounded to half, in out's type: the head's D features (of the DK computed) ----
     const float inv = 1.0f / attn_pair_sum(l);

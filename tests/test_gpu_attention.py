@@ -88,6 +88,24 @@ def test_attention(dev_sage, dev_16, sage, dt, out_dt, S, H, D, pad):
     check(got, want, out_dt, f"{'int8' if sage else '16-bit'} S={S} H={H} D={D}")
 
 
+@pytest.mark.parametrize("dt", [o.BF16, o.F16, o.F32])
+@pytest.mark.parametrize("L,Hq,Hkv,D,pad", [(512, 4, 2, 128, 0), (513, 8, 8, 128, 8), (577, 3, 1, 64, 0), (640, 2, 1, 96, 0), (705, 5, 1, 128, 3),
+                                            (1090, 16, 4, 64, 0), (511, 4, 1, 128, 0), (700, 33, 3, 64, 0)])
+def test_attention_causal_groups(dev, dt, L, Hq, Hkv, D, pad):
+    """From 512 rows and at most 32 heads (256 CUs) a block's wavefronts share its key tiles in two groups: odd and even
+    numbers of tiles, a group without a last tile, heads padded to the kernel's size, rows off 16-byte boundaries (q
+    prepared), and one case on either side of the line."""
+    qs, kvs = Hq * D + pad, 2 * Hkv * D + pad
+    g = np.random.default_rng(L)
+    q = o.to_dt(g.standard_normal((L, qs)).astype(np.float32), dt).ravel()
+    kv = o.to_dt(g.standard_normal((L, kvs)).astype(np.float32), dt).ravel()
+    want = o.attention_causal(q, kv, kv[Hkv * D:], dt, L, Hq, Hkv, D, qs, kvs)
+    qt, kvt = up(dev, q, DTS[dt], [L, qs]), up(dev, kv, DTS[dt], [L, kvs])
+    out = new(dev, DTS[dt], [L, Hq * D])
+    ops.attention_causal(ops.Rows(qt, 0, qs, L, Hq, D), ops.Rows(kvt, 0, kvs, L, Hkv, D), ops.Rows(kvt, Hkv * D, kvs, L, Hkv, D), out)
+    check(out.to_numpy().ravel(), want, dt, f"causal L={L} Hq={Hq} Hkv={Hkv} D={D}")
+
+
 @pytest.mark.parametrize("sage", [True, False])
 @pytest.mark.parametrize("S,pad", [(1, 0), (63, 2), (65, 0), (200, 6), (129, 1)])
 def test_attention_edges(dev_sage, dev_16, sage, S, pad):
