@@ -84,6 +84,26 @@ def test_int8_quantize_4096_pairs(request, layout):
     codes_close(q.to_numpy(), want_q, "codes")
 
 
+# ---- either side of the row counts from which the default context takes the one-wavefront-a-row layouts ----
+@pytest.mark.parametrize("C,M,tables", [(5376, 1023, "rows"), (5376, 1024, "rows"), (5376, 1025, None), (4096, 3071, None),
+                                        (4096, 3072, None), (4096, 3077, "one"), (4096, 3072, "rows"), (2048, 3073, "one")])
+def test_norm_quant_layout_lines(dev, C, M, tables):
+    rot, group = (o.ROT_REGULAR, 256) if C == DH else (o.ROT_SYLVESTER, 128)
+    rng = np.random.default_rng(C + M)
+    x, w = bf16_rows(C + M, M, C), (1 + 0.1 * rng.standard_normal(C)).astype(np.float32)
+    n = {"rows": 2, "one": 1}.get(tables, 0)
+    sc, sh = (0.1 * rng.standard_normal((2, n, C))).astype(np.float32) if n else (None, None)
+    rows = dit_rows(M) if tables == "rows" else None
+    want_q, want_s = o.norm_quant(x, o.BF16, M, C, w, 1e-5, rows, sc, sh, o.F32, o.BF16, rot, group)
+    tb = None
+    if n:
+        tb = ops.Tables(scale=up(dev, sc, "F32", [n, C]), shift=up(dev, sh, "F32", [n, C]), rows=up(dev, rows, "I32", [M]) if rows is not None else None)
+    q, s = new(dev, "I8", [M, C]), new(dev, "F32", [M])
+    ops.norm_quant(up(dev, x, "BF16", [M, C]), up(dev, w, "F32", [C]), 1e-5, tb, q, s, rot=rot, group=group)
+    assert_bits_equal(s.to_numpy(), want_s, "scales")
+    codes_close(q.to_numpy(), want_q, "codes")
+
+
 @pytest.mark.parametrize("layout", ["four", "wave"])
 def test_swiglu_quant_8192_pairs(request, layout):
     dev = request.getfixturevalue("dev" if layout == "four" else "dev_wave")
