@@ -12,7 +12,7 @@
 // bytes 16 (l / 32) .. + 15 of the slice) and the same 32 x 32 accumulator layout, so the operand path below works
 // in bytes and serves both: GemmArgs::K is the bytes of a row.
 //
-// Block: 512 threads (eight wavefronts, 2 x 4, two a SIMD), a 256 x 256 tile of out; each wavefront 128 x 64 as
+// Block: 512 threads (eight wavefronts, 2 x 4, two a SIMD), a 256 x 256 tile of out (or 192 x 256 or 128 x 256: gemm_plan); each wavefront 128 x 64 as
 // 4 x 2 v_mfma_i32_32x32x32_i8 accumulators (128 registers): while one wavefront of a SIMD waits (its fragment reads,
 // the step's barrier, its refill loads) the other issues products (four wavefronts of 128 x 128, one a SIMD, ran 6 %
 // slower; sixteen of 64 x 64, four a SIMD, 1.5 % slower). K advances 128 bytes a step (four
@@ -33,7 +33,7 @@
 // panels in its L2.
 // Epilogue: per 32-row slice of a wavefront's region, dequant + activation in registers, the slice through LDS,
 // then 16-byte row-contiguous stores (h3s_linear_acc: the slice in float32, the old output added as it is stored).
-// Split tiles (gemm_plan_split): a short last round of long-K tiles, or every tile of a launch of few tiles, runs
+// Split tiles (gemm_plan_split; 256 rows only): a short last round of long-K tiles, or every tile of a launch of few tiles, runs
 // as several blocks of consecutive K steps that leave their accumulators in scratch; gemm_merge_kernel sums them in
 // part order and applies the same epilogue arithmetic (gemm_values).
 #pragma once
@@ -45,16 +45,19 @@
 namespace h3 {
 
 constexpr int kGemmBM = 256, kGemmBN = 256, kGemmBK = 128, kGemmStages = 2;
-// Each wavefront computes kGemmWM rows x kGemmWN columns of the tile: kGemmWI x kGemmWJ accumulators of 32 x 32,
-// kGemmMF products a 32-deep slice, kGemmLoads direct loads of each operand a stage.
-constexpr int kGemmWM = 128, kGemmWN = 64, kGemmWI = kGemmWM / 32, kGemmWJ = kGemmWN / 32, kGemmMF = kGemmWI * kGemmWJ;
-constexpr int kGemmWaves = (kGemmBM / kGemmWM) * (kGemmBN / kGemmWN), kGemmThreads = 64 * kGemmWaves;
-constexpr int kGemmLoads = 32 / kGemmWaves;
-constexpr int kGemmStageBytes = (kGemmBM + kGemmBN) * kGemmBK;   // 64 KiB
-// the two stages, or the epilogue's scales and per-wavefront 32-row slices of float32 outputs, if larger
-constexpr int kGemmEpiBytes = 3 * 1024 + kGemmWaves * 32 * (kGemmWN * 4 + 16);
-constexpr int kGemmLds = kGemmStages * kGemmStageBytes > kGemmEpiBytes ? kGemmStages * kGemmStageBytes : kGemmEpiBytes;
-constexpr int kGemmTileAcc = kGemmBM * kGemmBN;                   // accumulators of a tile (a split tile's part)
+constexpr int kGemmWN = 64, kGemmWJ = kGemmWN / 32, kGemmWaves = 8, kGemmThreads = 64 * kGemmWaves;
+// A tile of 64 WI rows (WI 4: kGemmBM): each wavefront computes WM = 32 WI rows x kGemmWN columns, WI x kGemmWJ
+// accumulators of 32 x 32, MF products a 32-deep slice, with LA direct loads of A and LW of W a stage.
+constexpr int kGemmLW = kGemmBN * kGemmBK / 1024 / kGemmWaves;
+template <int WI> struct GemmTile {
+    static constexpr int BM = 64 * WI, WM = 32 * WI, MF = WI * kGemmWJ, LA = WI, LOADS = LA + kGemmLW;
+    static constexpr int STAGE = (BM + kGemmBN) * kGemmBK;       // 64 KiB of 256 rows
+    static_assert(BM * kGemmBK == LA * kGemmWaves * 1024, "GemmTile: A's loads");
+    // the two stages, or the epilogue's scales and per-wavefront 32-row slices of float32 outputs, if larger
+    static constexpr int EPI = 3 * 1024 + kGemmWaves * 32 * (kGemmWN * 4 + 16);
+    static constexpr int LDS = kGemmStages * STAGE > EPI ? kGemmStages * STAGE : EPI;
+};
+constexpr int kGemmTileAcc = kGemmBM * kGemmBN;                   // accumulators of a tile of 256 rows (a split tile's part)
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
@@ -165,12 +168,14 @@ __device__ __forceinline__ void gemm_values(const E (&a)[4], float sr, float f1,
 }
 
 // The kernel body for the operand type OP; ACC (16-bit operands only): out += the product.
-template <int OP, int ACT, bool PER_N, bool ACC>
+template <int OP, int ACT, bool PER_N, bool ACC, int WI = 4>
 __device__ __forceinline__ void gemm_body(const GemmArgs& P) {
     static_assert(OP == GEMM_I8 || (ACT == H3S_ACT_NONE && !PER_N), "gemm_body: the float epilogue has no scales or activation");
     static_assert(!ACC || OP != GEMM_I8, "gemm_body: accumulation into out is the float linear's");
     using Acc = std::conditional_t<OP == GEMM_I8, v16i, v16f>;
-    __shared__ __attribute__((aligned(16))) int8_t lds[kGemmLds];
+    using T = GemmTile<WI>;
+    constexpr int BM = T::BM, WM = T::WM, MF = T::MF;
+    __shared__ __attribute__((aligned(16))) int8_t lds[T::LDS];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / (kGemmBN / kGemmWN), wn = wave % (kGemmBN / kGemmWN);
     const int64_t K = P.K;
@@ -187,48 +192,51 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& P) {
         ke = (p + 1) * nk / P.split;
         part = u * P.split + p;
     }
-    const int64_t m0 = (int64_t) im * kGemmBM, n0 = (int64_t) in * kGemmBN;
+    const int64_t m0 = (int64_t) im * BM, n0 = (int64_t) in * kGemmBN;
     const bool half_last = K % kGemmBK != 0 && ke == nk;
-    // Instruction q of wavefront w fills units 64 (4 w + q) .. + 63: rows 8 (4 w + q) + lane / 8, each lane the
+    // Instruction q of wavefront w fills units 64 (L w + q) .. + 63 (L loads of the operand): rows 8 (L w + q) + lane / 8, each lane the
     // chunk its unit holds, so one instruction reads 8 whole 128-byte segments. The loads go through buffer resources
     // (gemm_rsrc): rows past the matrix's end read zeros (their products are not stored), so the lanes' 32-bit offsets
-    // are the same for both operands and every step, four registers, where clamped 64-bit addresses held 60 more
+    // are the same for every step (and, with 256 rows, for both operands), four registers, where clamped 64-bit addresses held 60 more
     // (196 registers against 256 and spills; 2 % faster). A half step's lanes of chunks 4-7 read the next row's first
     // bytes, or zeros after the last row; the slices that would use them are not run.
-    uint32_t vo[kGemmLoads];
+    uint32_t va[T::LA], vo[kGemmLW];
+    auto offset = [&](int first) {
+        const int r = 8 * first + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+        return (uint32_t) (r * K + 16 * c);
+    };
 #pragma unroll
-    for (int q = 0; q < kGemmLoads; ++q) {
-        const int r = 8 * (kGemmLoads * wave + q) + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
-        vo[q] = (uint32_t) (r * K + 16 * c);
-    }
+    for (int q = 0; q < T::LA; ++q) va[q] = offset(T::LA * wave + q);
+#pragma unroll
+    for (int q = 0; q < kGemmLW; ++q) vo[q] = offset(kGemmLW * wave + q);
     auto issue = [&](int kt) {
-        int8_t* st = lds + (kt % kGemmStages) * kGemmStageBytes;
+        int8_t* st = lds + (kt % kGemmStages) * T::STAGE;
         const int64_t k0 = (int64_t) kt * kGemmBK;
         const __amdgpu_buffer_rsrc_t ra = gemm_rsrc(P.A + m0 * K, P.M - m0, K, k0);
         const __amdgpu_buffer_rsrc_t rw = gemm_rsrc(P.W + n0 * K, P.N - n0, K, k0);
 #pragma unroll
-        for (int q = 0; q < kGemmLoads; ++q)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void*) (st + (kGemmLoads * wave + q) * 1024),
-                                                     16, vo[q], 0, 0, 0);
+        for (int q = 0; q < T::LA; ++q)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void*) (st + (T::LA * wave + q) * 1024),
+                                                     16, va[q], 0, 0, 0);
 #pragma unroll
-        for (int q = 0; q < kGemmLoads; ++q)
+        for (int q = 0; q < kGemmLW; ++q)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rw, (__attribute__((address_space(3))) void*) (st + kGemmBM * kGemmBK + (kGemmLoads * wave + q) * 1024), 16, vo[q], 0, 0, 0);
+                rw, (__attribute__((address_space(3))) void*) (st + BM * kGemmBK + (kGemmLW * wave + q) * 1024), 16, vo[q], 0, 0, 0);
     };
 
     // the epilogue's row and column scales, loaded now (three registers through the K steps) so that their latency
     // is not waited for at the end
     float sv = 0.0f, wv = 0.0f, bv = 0.0f;
-    if (tid < kGemmBM) {
+    if (tid < kGemmBN) {
         const int64_t m = m0 + tid < P.M ? m0 + tid : P.M - 1, n = n0 + tid < P.N ? n0 + tid : P.N - 1;
         if constexpr (OP == GEMM_I8) sv = P.sA[m];
         if constexpr (PER_N) wv = P.ws[n];
         if (P.bias) bv = P.bias[n];
     }
 
-    Acc acc[kGemmWI][kGemmWJ];
+    Acc acc[WI][kGemmWJ];
 #pragma unroll
-    for (int i = 0; i < kGemmWI; ++i)
+    for (int i = 0; i < WI; ++i)
 #pragma unroll
         for (int j = 0; j < kGemmWJ; ++j) acc[i][j] = (Acc) 0;
 
@@ -238,22 +246,22 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& P) {
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
         const int c = 2 * kk + (lane >> 5);
-        offA[kk] = gemm_unit(wm * kGemmWM + (lane & 31), c) * 16;
-        offW[kk] = kGemmBM * kGemmBK + gemm_unit(wn * kGemmWN + (lane & 31), c) * 16;
+        offA[kk] = gemm_unit(wm * WM + (lane & 31), c) * 16;
+        offW[kk] = BM * kGemmBK + gemm_unit(wn * kGemmWN + (lane & 31), c) * 16;
     }
 
-    // the fragments of one 32-deep slice kk of stage kt (kGemmWI of A and kGemmWJ of W)
-    auto read_half = [&](int kt, int kk, v4i (&a)[kGemmWI], v4i (&b)[kGemmWJ]) {
-        const int8_t* st = lds + (kt % kGemmStages) * kGemmStageBytes;
+    // the fragments of one 32-deep slice kk of stage kt (WI of A and kGemmWJ of W)
+    auto read_half = [&](int kt, int kk, v4i (&a)[WI], v4i (&b)[kGemmWJ]) {
+        const int8_t* st = lds + (kt % kGemmStages) * T::STAGE;
 #pragma unroll
-        for (int i = 0; i < (kGemmWI > kGemmWJ ? kGemmWI : kGemmWJ); ++i) {
-            if (i < kGemmWI) a[i] = *reinterpret_cast<const v4i*>(st + offA[kk] + 4096 * i);
+        for (int i = 0; i < (WI > kGemmWJ ? WI : kGemmWJ); ++i) {
+            if (i < WI) a[i] = *reinterpret_cast<const v4i*>(st + offA[kk] + 4096 * i);
             if (i < kGemmWJ) b[i] = *reinterpret_cast<const v4i*>(st + offW[kk] + 4096 * i);
         }
     };
     // W's fragment as the first operand: acc[i][j] holds rows (columns of out) from W tile j and columns (rows of
     // out) from A tile i, so each lane ends with four consecutive output columns of one output row per register group
-    auto mfma = [&](const v4i (&a)[kGemmWI], const v4i (&b)[kGemmWJ], int p) {
+    auto mfma = [&](const v4i (&a)[WI], const v4i (&b)[kGemmWJ], int p) {
         const int i = p / kGemmWJ, j = p % kGemmWJ;
         if constexpr (OP == GEMM_I8) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(b[j], a[i], acc[i][j], 0, 0, 0);
         else if constexpr (OP == GEMM_BF16)
@@ -265,21 +273,21 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& P) {
     };
     int issued = kb;
     for (; issued < kb + kGemmStages && issued < ke; ++issued) issue(issued);
-    v4i xa[kGemmWI], xb[kGemmWJ], ya[kGemmWI], yb[kGemmWJ];
-    if (issued - kb > 1) wait_vm<2 * kGemmLoads>(); else wait_vm<0>();
+    v4i xa[WI], xb[kGemmWJ], ya[WI], yb[kGemmWJ];
+    if (issued - kb > 1) wait_vm<T::LOADS>(); else wait_vm<0>();
     block_barrier();
     read_half(kb, 0, xa, xb);
-    // a slice's products (kGemmMF) with the next slice's fragment reads (kGemmWI + kGemmWJ) between them
-    auto body16 = [&](const v4i (&a)[kGemmWI], const v4i (&b)[kGemmWJ]) {
-        constexpr int NR = kGemmWI + kGemmWJ;
+    // a slice's products (MF) with the next slice's fragment reads (WI + kGemmWJ) between them
+    auto body16 = [&](const v4i (&a)[WI], const v4i (&b)[kGemmWJ]) {
+        constexpr int NR = WI + kGemmWJ;
 #pragma unroll
-        for (int p = 0; p < kGemmMF; ++p) mfma(a, b, p);
+        for (int p = 0; p < MF; ++p) mfma(a, b, p);
 #pragma unroll
-        for (int g = 0; g < (NR < kGemmMF ? NR : kGemmMF); ++g) {
+        for (int g = 0; g < (NR < MF ? NR : MF); ++g) {
             __builtin_amdgcn_sched_group_barrier(0x0008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x0100, NR <= kGemmMF ? 1 : (NR + kGemmMF - 1) / kGemmMF, 0);
+            __builtin_amdgcn_sched_group_barrier(0x0100, NR <= MF ? 1 : (NR + MF - 1) / MF, 0);
         }
-        if constexpr (kGemmMF > NR) __builtin_amdgcn_sched_group_barrier(0x0008, kGemmMF - NR, 0);
+        if constexpr (MF > NR) __builtin_amdgcn_sched_group_barrier(0x0008, MF - NR, 0);
     };
     // a step with the refill of stage kt + 2 (all but the last two steps) or without it, so that the loads sit in
     // the same scheduling region as the products they are interleaved with
@@ -291,7 +299,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& P) {
         body16(ya, yb);
         read_half(kt, 3, ya, yb);
         body16(xa, xb);
-        constexpr int PRE = kGemmMF / 4;      // the last slice's products before the barrier
+        constexpr int PRE = MF / 4;      // the last slice's products before the barrier
 #pragma unroll
         for (int p = 0; p < PRE; ++p) mfma(ya, yb, p);
         __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
@@ -300,18 +308,18 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& P) {
         if constexpr (REFILL) issue(kt + 2);
         read_half(kt + 1, 0, xa, xb);
 #pragma unroll
-        for (int p = PRE; p < kGemmMF; ++p) mfma(ya, yb, p);
+        for (int p = PRE; p < MF; ++p) mfma(ya, yb, p);
         // the rest of the slice's products, with the refill loads and the next stage's first fragment reads between them
         if constexpr (REFILL) {
 #pragma unroll
-            for (int g = 0; g < kGemmMF - PRE; ++g) {
+            for (int g = 0; g < MF - PRE; ++g) {
                 __builtin_amdgcn_sched_group_barrier(0x0008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x0020, (2 * kGemmLoads + kGemmMF - PRE - 1) / (kGemmMF - PRE), 0);
+                __builtin_amdgcn_sched_group_barrier(0x0020, (T::LOADS + MF - PRE - 1) / (MF - PRE), 0);
                 __builtin_amdgcn_sched_group_barrier(0x0100, 1, 0);
             }
         } else {
 #pragma unroll
-            for (int g = 0; g < kGemmMF - PRE; ++g) {
+            for (int g = 0; g < MF - PRE; ++g) {
                 __builtin_amdgcn_sched_group_barrier(0x0008, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x0100, 1, 0);
             }
@@ -330,18 +338,18 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& P) {
         body16(xa, xb);
     }
 #pragma unroll
-    for (int p = 0; p < kGemmMF; ++p) mfma(ya, yb, p);
+    for (int p = 0; p < MF; ++p) mfma(ya, yb, p);
     wait_vm<0>();
     if (part >= 0) {
         // a part of a split tile: its accumulators, register by register, 64 lanes' 4-byte values contiguous
         using E = std::conditional_t<OP == GEMM_I8, int, float>;
         // (the 32 x 32 blocks wholly past out's last row or column are not stored: the merge reads none of them)
-        E* dst = reinterpret_cast<E*>(P.part) + (size_t) part * kGemmTileAcc + wave * (kGemmMF * 16 * 64) + lane;
+        E* dst = reinterpret_cast<E*>(P.part) + (size_t) part * kGemmTileAcc + wave * (MF * 16 * 64) + lane;
 #pragma unroll
-        for (int i = 0; i < kGemmWI; ++i)
+        for (int i = 0; i < WI; ++i)
 #pragma unroll
             for (int j = 0; j < kGemmWJ; ++j) {
-                if (m0 + wm * kGemmWM + 32 * i >= P.M || n0 + wn * kGemmWN + 32 * j >= P.N) continue;
+                if (m0 + wm * WM + 32 * i >= P.M || n0 + wn * kGemmWN + 32 * j >= P.N) continue;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) dst[((i * kGemmWJ + j) * 16 + r) * 64] = acc[i][j][r];
             }
@@ -355,10 +363,10 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& P) {
     // Per 32-row slice i of this wavefront's 128 x 64 region: dequant + activation in registers, the four columns
     // as one 8-byte (16-bit out) or 16-byte (float32 out) LDS write, then 16-byte row-contiguous global stores.
     // One wavefront writes and reads its own slice, and a wavefront's LDS operations run in order.
-    float* srow = reinterpret_cast<float*>(lds);            // s[m] of the block's 256 rows
-    float* wcol = srow + kGemmBM;                           // wscale[n] of its 256 columns
+    float* srow = reinterpret_cast<float*>(lds);            // s[m] of the block's rows
+    float* wcol = srow + kGemmBN;                           // wscale[n] of its 256 columns
     float* bcol = wcol + kGemmBN;                           // bias[n]
-    if (tid < kGemmBM) {
+    if (tid < kGemmBN) {
         srow[tid] = sv;
         wcol[tid] = wv;
         bcol[tid] = bv;
@@ -375,7 +383,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& P) {
         int8_t* slice = lds + 3 * 1024 + wave * (32 * pitch);
         const float ws0 = OP == GEMM_I8 && !PER_N ? P.ws[0] : 0.0f;
         // rows of out start on 16-byte boundaries and the block's tile lies inside out: plain 16-byte stores
-        const bool full = (P.N * esz) % 16 == 0 && m0 + kGemmBM <= P.M && n0 + kGemmBN <= P.N;
+        const bool full = (P.N * esz) % 16 == 0 && m0 + BM <= P.M && n0 + kGemmBN <= P.N;
         constexpr int per_row = kGemmWN * esz / 16, epc = 16 / esz, kpl = 32 * per_row / 64;
         // h3s_linear_acc on a tile inside out: the old output of a slice's pieces loaded a slice ahead (slice 0's
         // before any arithmetic), so their latency passes under a slice's work instead of stalling its stores
@@ -384,7 +392,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& P) {
 #pragma unroll
             for (int k = 0; k < kpl; ++k) {
                 const int ch = lane + 64 * k, rr = ch / per_row, cg = ch % per_row;
-                const int64_t m = m0 + wm * kGemmWM + i * 32 + rr, n = n0 + wn * kGemmWN + (int64_t) cg * epc;
+                const int64_t m = m0 + wm * WM + i * 32 + rr, n = n0 + wn * kGemmWN + (int64_t) cg * epc;
                 d[k] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(P.out) + (m * P.N + n) * esz);
             }
         };
@@ -392,8 +400,8 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& P) {
             if (full) load_old(0, oldv[0]);
         }
 #pragma unroll
-        for (int i = 0; i < kGemmWI; ++i) {
-            const float sr = srow[wm * kGemmWM + i * 32 + (lane & 31)];
+        for (int i = 0; i < WI; ++i) {
+            const float sr = srow[wm * WM + i * 32 + (lane & 31)];
             const float f1 = sr * ws0;
 #pragma unroll
             for (int j = 0; j < kGemmWJ; ++j)
@@ -421,9 +429,9 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& P) {
                     else
                         *reinterpret_cast<uint2*>(at) = make_uint2(pack_f16(v[0], v[1]), pack_f16(v[2], v[3]));
                 }
-            const int64_t mt = m0 + wm * kGemmWM + i * 32, nt = n0 + wn * kGemmWN;
+            const int64_t mt = m0 + wm * WM + i * 32, nt = n0 + wn * kGemmWN;
             if constexpr (ACC) {
-                if (full && i + 1 < kGemmWI) load_old(i + 1, oldv[(i + 1) & 1]);
+                if (full && i + 1 < WI) load_old(i + 1, oldv[(i + 1) & 1]);
                 // each 16-byte piece of a row of out: its epc staged values + the old ones, rounded once
 #pragma unroll
                 for (int k = 0; k < kpl; ++k) {
@@ -487,14 +495,14 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& P) {
     else { if (P.bias) epilogue(f32_t{}, yes{}); else epilogue(f32_t{}, no{}); }
 }
 
-template <int ACT, bool PER_N>
+template <int ACT, bool PER_N, int WI>
 __global__ __launch_bounds__(kGemmThreads, 1) void gemm_i8_kernel(GemmArgs P) {
-    gemm_body<GEMM_I8, ACT, PER_N, false>(P);
+    gemm_body<GEMM_I8, ACT, PER_N, false, WI>(P);
 }
 // the float linear: 16-bit operands (OP GEMM_BF16 or GEMM_F16), out = x w^T [+ bias] (ACC: out += x w^T [+ bias])
-template <int OP, bool ACC>
+template <int OP, bool ACC, int WI>
 __global__ __launch_bounds__(kGemmThreads, 1) void gemm_f16_kernel(GemmArgs P) {
-    gemm_body<OP, H3S_ACT_NONE, false, ACC>(P);
+    gemm_body<OP, H3S_ACT_NONE, false, ACC, WI>(P);
 }
 
 // The split tiles' epilogue: a thread takes one group of four accumulators of a tile (the wavefront, 32 x 32 block,
@@ -506,16 +514,16 @@ __global__ __launch_bounds__(256) void gemm_merge_kernel(GemmArgs P) {
     using E = std::conditional_t<OP == GEMM_I8, int, float>;
     const int u = (int) blockIdx.x / kGemmMergeBlocks;
     const int t = ((int) blockIdx.x % kGemmMergeBlocks) * 256 + (int) threadIdx.x;
-    const int lane = t & 63, grp = t >> 6;              // grp = ((wave kGemmWI + i) kGemmWJ + j) 4 + g
-    const int g = grp & 3, j = (grp >> 2) % kGemmWJ, i = (grp >> 2) / kGemmWJ % kGemmWI, wave = (grp >> 2) / kGemmMF;
+    const int lane = t & 63, grp = t >> 6;              // grp = ((wave 4 + i) kGemmWJ + j) 4 + g
+    const int g = grp & 3, j = (grp >> 2) % kGemmWJ, i = (grp >> 2) / kGemmWJ % 4, wave = (grp >> 2) / (4 * kGemmWJ);
     const int wm = wave / (kGemmBN / kGemmWN), wn = wave % (kGemmBN / kGemmWN);
     int im, in;
     gemm_tile_of(P.main_tiles + u, P.tm, P.tn, P.gh, &im, &in);
-    const int64_t m = (int64_t) im * kGemmBM + wm * kGemmWM + i * 32 + (lane & 31);
+    const int64_t m = (int64_t) im * kGemmBM + wm * 128 + i * 32 + (lane & 31);
     const int64_t n = (int64_t) in * kGemmBN + wn * kGemmWN + j * 32 + 8 * g + 4 * (lane >> 5);
     if (m >= P.M || n >= P.N) return;
     const E* src = reinterpret_cast<const E*>(P.part) + (size_t) u * P.split * kGemmTileAcc +
-                   ((wave * kGemmWI + i) * kGemmWJ + j) * 16 * 64 + 4 * g * 64 + lane;
+                   ((wave * 4 + i) * kGemmWJ + j) * 16 * 64 + 4 * g * 64 + lane;
     E a[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) a[q] = src[q * 64];
@@ -569,6 +577,43 @@ inline void gemm_plan_split(int64_t tiles, int64_t nk, int cus, int* main_tiles,
     if (narrow && 24 * nk * (s - 1) <= rem * s * s + 60 * s) return;
     *main_tiles = (int) full;
     *split = (int) s;
+}
+
+// The height of a launch's tiles (64 wi rows: 256, 192 or 128) and their split (256-row tiles only; may_split false: none).
+// 256 rows read the fewest bytes a product and run full rounds of the device fastest, but a launch of few rounds pays for
+// its last one: the estimate below, in microseconds a K step (a full round of 256 CUs; a last round's CUs also run faster the
+// fewer they are, from `least` up to a full round's, as the square of its share), is within about 8 % of the measured times
+// of the DiT's four int8 linears at 256 .. 16896 rows, and a lower tile is taken where it says 3 % or more. Measured, 256
+// rows against the choice: 7168 -> 5376 at 2159 rows 78.9 -> 75.7 us (189 tiles, 252), at 1500 82.1 -> 57.7, at 4096
+// 160 -> 142; 14336 -> 5376 at 2159 152 -> 146; 5376 -> 28672 at 300 62.4 -> 54.7, at 3000 448 -> 420. (16-bit operands
+// 5376 -> 14336, cold weights: 640 rows 123 -> 112, 768 128 -> 121, 520 115 -> 117.) A split launch's parts
+// are written and read at about 0.1 us a part of 256 live rows. Short products (below 32 steps) keep 256 rows: there the
+// epilogue, not the steps, is the time.
+struct GemmPlan { int wi, main_tiles, split; };
+inline double gemm_round_us(int64_t tiles, int wi, int cus) {
+    const double full = wi == 4 ? 1.75 : wi == 3 ? 1.33 : 1.0, least = wi == 4 ? 1.05 : wi == 3 ? 0.95 : 0.82;
+    const double f = (double) (tiles % cus) / cus;
+    return (double) (tiles / cus) * full + (f > 0.0 ? least + (full - least) * f * f : 0.0);
+}
+inline GemmPlan gemm_plan(int64_t M, int64_t N, int64_t nk, int cus, bool may_split) {
+    const int64_t tn = (N + kGemmBN - 1) / kGemmBN, tm = (M + kGemmBM - 1) / kGemmBM, tiles = tm * tn;
+    GemmPlan p{4, (int) tiles, 1};
+    if (may_split) gemm_plan_split(tiles, nk, cus, &p.main_tiles, &p.split);
+    if (nk < 32) return p;
+    double us = gemm_round_us(p.main_tiles, 4, cus) * (double) nk;
+    if (p.split > 1) {
+        const int64_t parts = (tiles - p.main_tiles) * p.split;
+        us += gemm_round_us(parts, 4, cus) * (double) ((nk + p.split - 1) / p.split) + 3.0 +
+              0.1 * (double) parts * (double) M / (double) (tm * kGemmBM);
+    }
+    us *= 0.97;
+    for (int wi = 3; wi >= 2; --wi) {
+        const int64_t t = (M + 64 * wi - 1) / (64 * wi) * tn;
+        if (t > 0x7fffffff) break;
+        const double u = gemm_round_us(t, wi, cus) * (double) nk;
+        if (u < us) { us = u; p = {wi, (int) t, 1}; }
+    }
+    return p;
 }
 
 }  // namespace h3

@@ -49,10 +49,11 @@ static void* scratch_on(int device, std::string& why) {
 // scratch, for the allocation-free entry point)
 int launch_gemm(Ctx* c, const char* fn, const int8_t* q, const float* s, int64_t M, int64_t K, const int8_t* w, int64_t N,
                 const float* wscale, int64_t n_wscale, const float* bias, int act_, void* out, int out_dt, bool split_ok) {
-    const int64_t tm = (M + kGemmBM - 1) / kGemmBM, tn = (N + kGemmBN - 1) / kGemmBN;
-    if (tm * tn > 0x7fffffff || tm > 0x7fffffff || tn > 0x7fffffff) return fail(std::string(fn) + ": too many tiles");
-    int main_tiles = (int) (tm * tn), split = 1;
-    if (split_ok) gemm_plan_split(tm * tn, (K + kGemmBK - 1) / kGemmBK, c->cus, &main_tiles, &split);
+    const int64_t tm0 = (M + kGemmBM - 1) / kGemmBM, tn = (N + kGemmBN - 1) / kGemmBN;
+    if (tm0 * tn > 0x7fffffff || tm0 > 0x7fffffff || tn > 0x7fffffff) return fail(std::string(fn) + ": too many tiles");
+    const GemmPlan plan = gemm_plan(M, N, (K + kGemmBK - 1) / kGemmBK, c->cus, split_ok);
+    const int wi = plan.wi, main_tiles = plan.main_tiles, split = plan.split;
+    const int64_t tm = (M + 64 * wi - 1) / (64 * wi);
     const int64_t tail = tm * tn - main_tiles;
     void* part = nullptr;
     if (split > 1) {
@@ -79,7 +80,9 @@ int launch_gemm(Ctx* c, const char* fn, const int8_t* q, const float* s, int64_t
     }
 #define LG(ACT, PN)                                                        \
     {                                                                      \
-        gemm_i8_kernel<ACT, PN><<<grid, kGemmThreads, 0, c->stream>>>(P);  \
+        if (wi == 2) gemm_i8_kernel<ACT, PN, 2><<<grid, kGemmThreads, 0, c->stream>>>(P);  \
+        else if (wi == 3) gemm_i8_kernel<ACT, PN, 3><<<grid, kGemmThreads, 0, c->stream>>>(P);  \
+        else gemm_i8_kernel<ACT, PN, 4><<<grid, kGemmThreads, 0, c->stream>>>(P);  \
         LM(ACT, PN)                                                        \
     }
 #define LA(ACT)                    \

@@ -106,9 +106,17 @@ static void merge_f16(Ctx* c, const GemmArgs& P, unsigned mgrid) {
 }
 static int linear_mfma(Ctx* c, const char* fn, const void* x, int dt, int64_t M, int64_t K, const void* w, int64_t N,
                        const float* bias, void* out, int out_dt, bool acc) {
-    const int64_t tm = (M + kGemmBM - 1) / kGemmBM, tn = (N + kGemmBN - 1) / kGemmBN, kb = 2 * K;
-    int main_tiles = (int) (tm * tn), split = 1;
-    gemm_plan_split(tm * tn, (kb + kGemmBK - 1) / kGemmBK, c->cus, &main_tiles, &split);
+    const int64_t tn = (N + kGemmBN - 1) / kGemmBN, kb = 2 * K;
+    GemmPlan plan{4, 0, 1};
+    if (acc) {
+        const int64_t tiles = (M + kGemmBM - 1) / kGemmBM * tn;
+        plan.main_tiles = (int) tiles;
+        gemm_plan_split(tiles, (kb + kGemmBK - 1) / kGemmBK, c->cus, &plan.main_tiles, &plan.split);
+    } else {
+        plan = gemm_plan(M, N, (kb + kGemmBK - 1) / kGemmBK, c->cus, true);
+    }
+    const int wi = plan.wi, main_tiles = plan.main_tiles, split = plan.split;
+    const int64_t tm = (M + 64 * wi - 1) / (64 * wi);
     const int64_t tail = tm * tn - main_tiles;
     void* part = nullptr;
     if (split > 1) {
@@ -119,12 +127,16 @@ static int linear_mfma(Ctx* c, const char* fn, const void* x, int dt, int64_t M,
                      kb >= 12288 ? 4 : 8, main_tiles, split, part};
     const unsigned grid = (unsigned) (main_tiles + tail * split), mgrid = (unsigned) (tail * kGemmMergeBlocks);
     if (dt == H3S_BF16) {
-        if (acc) gemm_f16_kernel<GEMM_BF16, true><<<grid, kGemmThreads, 0, c->stream>>>(P);
-        else gemm_f16_kernel<GEMM_BF16, false><<<grid, kGemmThreads, 0, c->stream>>>(P);
+        if (acc) gemm_f16_kernel<GEMM_BF16, true, 4><<<grid, kGemmThreads, 0, c->stream>>>(P);
+        else if (wi == 2) gemm_f16_kernel<GEMM_BF16, false, 2><<<grid, kGemmThreads, 0, c->stream>>>(P);
+        else if (wi == 3) gemm_f16_kernel<GEMM_BF16, false, 3><<<grid, kGemmThreads, 0, c->stream>>>(P);
+        else gemm_f16_kernel<GEMM_BF16, false, 4><<<grid, kGemmThreads, 0, c->stream>>>(P);
         if (split > 1) { if (acc) merge_f16<GEMM_BF16, true>(c, P, mgrid); else merge_f16<GEMM_BF16, false>(c, P, mgrid); }
     } else {
-        if (acc) gemm_f16_kernel<GEMM_F16, true><<<grid, kGemmThreads, 0, c->stream>>>(P);
-        else gemm_f16_kernel<GEMM_F16, false><<<grid, kGemmThreads, 0, c->stream>>>(P);
+        if (acc) gemm_f16_kernel<GEMM_F16, true, 4><<<grid, kGemmThreads, 0, c->stream>>>(P);
+        else if (wi == 2) gemm_f16_kernel<GEMM_F16, false, 2><<<grid, kGemmThreads, 0, c->stream>>>(P);
+        else if (wi == 3) gemm_f16_kernel<GEMM_F16, false, 3><<<grid, kGemmThreads, 0, c->stream>>>(P);
+        else gemm_f16_kernel<GEMM_F16, false, 4><<<grid, kGemmThreads, 0, c->stream>>>(P);
         if (split > 1) { if (acc) merge_f16<GEMM_F16, true>(c, P, mgrid); else merge_f16<GEMM_F16, false>(c, P, mgrid); }
     }
     return launched(fn);

@@ -65,6 +65,22 @@ def test_int8_gemm_split(dev4, M, K, N, per_n, bias, out_dt, act):
         assert_close_16(out.to_numpy(), want, out_dt, "gemm split silu", max_frac=5e-3)
 
 
+# launches of few rounds take tiles of 192 or 128 rows (gemm_plan, for 4 compute units): (192) 2 x 3 tiles with a half step,
+# 2 x 2 whole tiles, one row of 4; (128) one row of 3 tiles, whole rows and a half step; and 256 rows with its split kept
+@pytest.mark.parametrize("per_n,bias,out_dt", [(False, False, o.BF16), (True, True, o.F32), (True, False, o.F16)])
+@pytest.mark.parametrize("M,K,N", [(260, 4160, 600), (384, 4096, 500), (190, 4224, 1000), (120, 4096, 600), (128, 4160, 700), (1, 4096, 601),
+                                   (500, 12288, 600)])
+def test_int8_gemm_tile_heights(dev4, M, K, N, per_n, bias, out_dt):
+    test_int8_gemm_split(dev4, M, K, N, per_n, bias, out_dt, o.ACT_NONE)
+
+
+# the same on 16-bit operands: 192 rows (3 x 2 tiles, a half step; 4 x 1), 128 rows (5 x 3), 256 rows with its split kept
+@pytest.mark.parametrize("dt,out_dt,bias", [(o.BF16, o.BF16, True), (o.F16, o.F32, False)])
+@pytest.mark.parametrize("M,K,N", [(520, 2080, 300), (640, 2048, 200), (640, 2080, 600), (1100, 6176, 200)])
+def test_linear_tile_heights(dev4, dt, out_dt, bias, M, K, N):
+    test_linear_split(dev4, dt, out_dt, M, K, N, bias)
+
+
 @pytest.mark.parametrize("group", [0, 256])
 def test_int8_linear_split(dev4, group):
     """h3s_int8_linear (the quantizer, then the GEMM with its last tiles split) against the oracle, bit for bit."""
