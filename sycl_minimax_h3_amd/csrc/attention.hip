@@ -11,7 +11,7 @@
 namespace h3 {
 
 // q of Hq heads (row stride qs) and k, v of Hkv heads (row stride kvs) prepared into aq [Hq, Sp, DK], ak [Hkv, Sp, DK]
-// (int8 codes with their scales for SAGE, else half) and av [Hkv, DK, Sp] (half), DK = attn_dk(D), zero past D
+// (int8 codes with their scales for SAGE, else half) and av [Hkv, Sp / 32, DK, 32] (half), DK = attn_dk(D), zero past D
 // (q_in_kernel: the attention kernel forms q's fragments from q itself, so q is not prepared)
 template <int DT>
 static void prep(Ctx* c, const void* q, const void* k, const void* v, int64_t S, int64_t Sp, int64_t Hq, int64_t Hkv, int D,

@@ -397,7 +397,7 @@ __global__ __launch_bounds__(256) void attn_kv_prep_vec_kernel(const void* __res
     else attn_v_prep_body<DT, D>(b - n, v, S, Sp, stride, vt);
 }
 
-// v of one head and 64 tokens to half, transposed: vt [H, DK, Sp]; tokens past S and features past D become zeros
+// v of one head and 64 tokens to half, transposed: vt [H, Sp / 32, DK, 32]; tokens past S and features past D become zeros
 template <int DT>
 __global__ __launch_bounds__(256) void attn_v_prep_kernel(const void* __restrict__ v, int64_t S, int64_t Sp, int D, int DK,
                                                           int64_t stride, uint16_t* __restrict__ vt) {
@@ -430,7 +430,7 @@ __device__ __forceinline__ void block_barrier_a() { asm volatile("s_barrier" :::
 struct AttnArgs {
     const int8_t* q;          // [H, Sp, D]: int8 codes (SAGE) or half bits
     const int8_t* k;
-    const uint16_t* vt;       // [H, D, Sp] half bits
+    const uint16_t* vt;       // [H, Sp / 32, D, 32] half bits (attn_vt_pos)
     const float* qs;          // [H, Sp / 64] (SAGE)
     const float* ks;
     int64_t S, Sp, H;
