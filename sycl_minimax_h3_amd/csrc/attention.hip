@@ -89,12 +89,12 @@ static int attention_one(Ctx* c, const char* fn, const void* q, const void* k, c
     if (Hq * (Sp / qblock) > 0x7fffffff) return fail(std::string(fn) + ": too many query blocks");
     // the wide kernel, and the 16-bit form of the others, read q's rows themselves where they are whole 16-byte vectors of
     // unpadded heads (no prepared q then: one launch less, and q neither written nor read again)
-    // (a block of the others then writes out while another may still read q: an out that overlaps q otherwise than row on
-    // row has q prepared first)
+    // (a block writes its rows of out when it ends, where others have yet to read their rows of q: an out that overlaps q
+    // otherwise than row on row has q prepared first. k and v are always prepared before any block runs.)
     const char *qb0 = (const char*) q, *ob0 = (const char*) out;
     const bool apart = ob0 + S * Hq * D * elem_size(out_dt) <= qb0 || qb0 + S * qs_stride * elem_size(dt) <= ob0 ||
                        (ob0 == qb0 && qs_stride == Hq * D && elem_size(dt) == elem_size(out_dt));
-    const bool q_in_kernel = (pp || (!sage && apart)) && D == DK && aligned16(q) && (qs_stride * elem_size(dt)) % 16 == 0;
+    const bool q_in_kernel = (pp || !sage) && apart && D == DK && aligned16(q) && (qs_stride * elem_size(dt)) % 16 == 0;
     int8_t* aq = q_in_kernel ? nullptr : c->scratch<int8_t>(Ctx::ATT_Q, (size_t) (Sp * Hq * DK * esz));
     const size_t over = pp ? kAttnOver : 0;                   // what its last direct loads read past the end
     int8_t* ak = c->scratch<int8_t>(Ctx::ATT_K, (size_t) (Sp * Hkv * DK * esz) + over);

@@ -1,5 +1,7 @@
 """Helpers shared by the tests: uploads, bit comparisons of 16-bit floats, and the parity tolerance for results
 through transcendental functions (relative error 1e-3, one unit in the last place on few elements)."""
+import ctypes
+
 import numpy as np
 
 from oracle import oracle as o
@@ -65,3 +67,55 @@ def codes_close(got_q, want_q, what=""):
     d = np.abs(np.asarray(got_q, dtype=np.int32).ravel() - np.asarray(want_q, dtype=np.int32).ravel())
     assert d.max(initial=0) <= 1, f"{what}: a code differs by {d.max()}"
     assert int((d > 0).sum()) == 0, f"{what}: {int((d > 0).sum())} codes differ by 1"
+
+
+class _Dim3(ctypes.Structure):
+    _fields_ = [("x", ctypes.c_uint32), ("y", ctypes.c_uint32), ("z", ctypes.c_uint32)]
+
+
+class _KernelNodeParams(ctypes.Structure):   # hipKernelNodeParams
+    _fields_ = [("block", _Dim3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", _Dim3),
+                ("params", ctypes.c_void_p), ("shared", ctypes.c_uint)]
+
+
+def launches(dev, call):
+    """The kernels `call` launches on the context's stream, in order, as (name with its template arguments, blocks, threads
+    a block): `call` runs once as it is (which grows the context's scratch), then once while the stream records a graph,
+    which is read and never launched."""
+    hip = dev.api.lib            # the library's own HIP runtime
+    vp, sz = ctypes.c_void_p, ctypes.c_size_t
+    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
+    hip.hipKernelNameRefByPtr.argtypes = [vp, vp]
+
+    def ok(rc, what):
+        assert rc == 0, f"{what}: HIP error {rc}"
+
+    call()
+    dev.wait()
+    stream, graph, n = vp(dev.stream()), vp(), sz(0)
+    ok(hip.hipStreamBeginCapture(stream, 2), "hipStreamBeginCapture")       # 2: relaxed
+    try:
+        call()
+    finally:
+        rc = hip.hipStreamEndCapture(stream, ctypes.byref(graph))
+    ok(rc, "hipStreamEndCapture")
+    out = []
+    try:
+        ok(hip.hipGraphGetNodes(graph, None, ctypes.byref(n)), "hipGraphGetNodes")
+        nodes = (vp * n.value)()
+        ok(hip.hipGraphGetNodes(graph, nodes, ctypes.byref(n)), "hipGraphGetNodes")
+        demangle = ctypes.CDLL("libstdc++.so.6").__cxa_demangle
+        demangle.restype, demangle.argtypes = ctypes.c_char_p, [ctypes.c_char_p, vp, vp, vp]
+        for node in nodes:
+            kind = ctypes.c_int(-1)
+            ok(hip.hipGraphNodeGetType(vp(node), ctypes.byref(kind)), "hipGraphNodeGetType")
+            assert kind.value == 0, f"a node of type {kind.value} that is no kernel launch"
+            p = _KernelNodeParams()
+            ok(hip.hipGraphKernelNodeGetParams(vp(node), ctypes.byref(p)), "hipGraphKernelNodeGetParams")
+            name = hip.hipKernelNameRefByPtr(p.func, stream) or b"?"
+            name = (demangle(name, None, None, None) or name).decode()
+            name = name.split("(h3::")[0].removeprefix("void ").replace("h3::", "")
+            out.append((name, p.grid.x * p.grid.y * p.grid.z, p.block.x))
+    finally:
+        ok(hip.hipGraphDestroy(graph), "hipGraphDestroy")
+    return out

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as o
-from helpers import new, up
+from helpers import launches, new, up
 
 pytestmark = pytest.mark.gpu
 
@@ -332,3 +332,42 @@ def test_attention_wide_split_ranges(dev_split, sage, dt):
     want = want[0] if sage else want
     got = run(dev_split[(sage, "default")], q, k, v, dt, S, H, D, H * D, o.F32)
     check(got, want, o.F32, f"wide split {sage}")
+
+
+@pytest.mark.parametrize("where", ["row on row", "in the q rows", "across q", "over k", "over v"])
+@pytest.mark.parametrize("form,dt,S,H,D", [("int8", o.BF16, 1100, 3, 128), ("16-bit", o.BF16, 1100, 3, 128), ("16-bit", o.F32, 900, 2, 128),
+                                           ("16-bit", o.F16, 600, 2, 64), ("int8", o.BF16, 600, 2, 64), ("causal", o.BF16, 1100, 3, 128),
+                                           ("causal", o.BF16, 300, 3, 64)])
+def test_attention_out_over_inputs(dev, dev_sage, dev_16, form, dt, S, H, D, where):
+    """out in memory that q, k or v also lie in: row on row with a contiguous q (each block has read its rows before it
+    writes them), and otherwise (q prepared first: the launches say so). q, k and v are the columns of one buffer, whose
+    rows out then runs along at a third of the stride, or contiguous tensors."""
+    d = {"int8": dev_sage, "16-bit": dev_16, "causal": dev}[form]
+    W = H * D
+    q, k, v = qkv(140 + S + D, S, H, D, dt, W)
+    if form == "causal":
+        want = o.attention_causal(q, k, v, dt, S, H, H, D, W, W)
+    else:
+        want = o.attention(q, k, v, dt, S, H, D, W, out_dt=dt, sage=form == "int8")
+        want = want[0] if form == "int8" else want
+    two = lambda a: a.reshape(S, W)  # noqa: E731
+    esz = DTS[dt].size()
+    if where == "in the q rows":                                 # q | k | v in rows of 3 W, out contiguous from the start
+        buf = up(d, np.concatenate([two(q), two(k), two(v)], 1).ravel(), DTS[dt], [S, 3 * W])
+        qr, kr, vr = (ops.Rows(buf, i * W, 3 * W, S, H, D) for i in range(3))
+        out = Tensor(DTS[dt], [S, W], buf.ptr(), buf._owner, d)
+    elif where == "across q":                                    # out starts 64 rows after q in one allocation
+        buf = up(d, np.concatenate([q, q[:64 * W]]), DTS[dt], [S + 64, W])
+        kt, vt = (up(d, a, DTS[dt], [S, W]) for a in (k, v))
+        qr, kr, vr = ops.Rows(buf, 0, W, S, H, D), ops.Rows(kt, 0, W, S, H, D), ops.Rows(vt, 0, W, S, H, D)
+        out = Tensor(DTS[dt], [S, W], buf.ptr() + 64 * W * esz, buf._owner, d)
+    else:
+        qt, kt, vt = (up(d, a, DTS[dt], [S, W]) for a in (q, k, v))
+        qr, kr, vr = (ops.Rows(t, 0, W, S, H, D) for t in (qt, kt, vt))
+        out = {"row on row": qt, "over k": kt, "over v": vt}[where]
+    call = lambda: (ops.attention_causal if form == "causal" else ops.attention)(qr, kr, vr, out)  # noqa: E731
+    call()
+    check(out.to_numpy().ravel(), want, dt, f"{form} out {where}")
+    names = [n for n, _, _ in launches(d, call)]                 # (on what the first call left: only the launches are read)
+    q_prepared = any("qk_prep" in n for n in names)
+    assert q_prepared == (where in ("in the q rows", "across q") or (form == "int8" and D == 64)), names
