@@ -637,15 +637,17 @@ __global__ __launch_bounds__(256 * KS, KS == 2 ? 2 : DK == 256 ? 1 : 3) void att
         if (__any(mx > m + 8.0f)) {
             asm volatile("" ::: "memory");
             const float mn = fmaxf(m, mx);
-            // (KS: a lane may have seen no live score yet, m = mn = -infinity)
-            const float alpha = KS > 1 && m == mn ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+            // (a lane may have seen no live score yet, m = mn = -infinity)
+            const float alpha = m == mn ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
             m = mn;
             l = l * alpha;
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt) o[dt] = o[dt] * alpha;
         }
+        // (scores of -infinity, an infinite k's, weigh nothing; before any other score m is still -infinity itself)
+        const float ref = m == -INFINITY ? 0.0f : m;
 #pragma unroll
-        for (int i = 0; i < 32; ++i) x[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[i], f, -m));
+        for (int i = 0; i < 32; ++i) x[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[i], f, -ref));
         if constexpr (TAIL) {
 #pragma unroll
             for (int i = 0; i < 32; ++i)
@@ -996,8 +998,8 @@ __global__ __launch_bounds__(256, 2) void attn_pl_kernel(AttnArgs P) {
             // The weights p = 2^(score f - m) rounded to half, packed as the P v products take them (chunk s: registers
             // 8 s .. 8 s + 7), and their sum over this lane's keys. SAGE: score f - m = x f - (kScoreBias f + m), with
             // one rounding of the offset (relative 2^-24 of kScoreBias f, far below half's rounding of p).
-            auto weights = [&]() {
-                const float c = SAGE ? __builtin_fmaf(kScoreBias, f, m[gq]) : m[gq];
+            auto weights = [&](float ref) {
+                const float c = SAGE ? __builtin_fmaf(kScoreBias, f, ref) : ref;
                 float ls[2];
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
@@ -1023,7 +1025,7 @@ __global__ __launch_bounds__(256, 2) void attn_pl_kernel(AttnArgs P) {
             // 16 above m, or m not yet set) rounds to infinity and makes the lane's sum infinite. Only then the tile's
             // max: m moves when it passes m by more than 8 (as in attn_kernel), O and l are rescaled and the weights
             // computed again (each at most 1 then). O / l does not depend on m.
-            float lt = weights();
+            float lt = weights(m[gq]);
             if (__any(!(lt <= 3.0e38f))) {
                 asm volatile("" ::: "memory");
                 float mt[8];
@@ -1045,7 +1047,9 @@ __global__ __launch_bounds__(256, 2) void attn_pl_kernel(AttnArgs P) {
 #pragma unroll
                     for (int dt = 0; dt < NDT; ++dt) o[gq][dt] = o[gq][dt] * alpha;
                 }
-                lt = weights();
+                // (a tile of scores that are all -infinity, an infinite k's, before any other: they weigh nothing, and m
+                // stays unset)
+                lt = weights(m[gq] == -INFINITY ? 0.0f : m[gq]);
             }
             l[gq] = l[gq] + lt;
             // slice gq's fragments of V^T, into the registers this group's scores leave

@@ -371,3 +371,56 @@ def test_attention_out_over_inputs(dev, dev_sage, dev_16, form, dt, S, H, D, whe
     names = [n for n, _, _ in launches(d, call)]                 # (on what the first call left: only the launches are read)
     q_prepared = any("qk_prep" in n for n in names)
     assert q_prepared == (where in ("in the q rows", "across q") or (form == "int8" and D == 64)), names
+
+
+@pytest.mark.parametrize("value", [-np.inf, -1e30])
+@pytest.mark.parametrize("form,dt,L,Hq,D,dead", [
+    ("causal", o.BF16, 600, 4, 128, [(64, 128)]),               # two key groups: the second group's first tile
+    ("causal", o.BF16, 700, 3, 64, [(64, 128), (192, 256)]),    # and a later one
+    ("causal", o.F32, 640, 2, 128, [(0, 63), (64, 128)]),       # nearly all of the first group's too
+    ("causal", o.BF16, 200, 2, 128, [(64, 128)]),               # one group
+    ("whole", o.BF16, 300, 2, 128, [(0, 32)]),                  # the wide form's first tile of 32 keys
+    ("whole", o.BF16, 1500, 2, 128, [(0, 40), (192, 256), (1470, 1500)]),   # the first tiles of split ranges
+    ("whole", o.F32, 300, 2, 64, [(0, 64), (250, 300)]),        # heads of 64: the first tile of 64 keys
+    ("whole", o.BF16, 150, 1, 256, [(0, 100)]),
+])
+def test_attention_dead_keys(dev, dev_16, form, dt, L, Hq, D, dead, value):
+    """Keys that every query scores at minus infinity (an infinite feature, or one past half's range: the operands are
+    half) weigh nothing, wherever the tiles of a walk over the keys begin: whole tiles of them, the first of a key group,
+    of a split range or of the walk itself among them."""
+    g = np.random.default_rng(L + D)
+    q, k, v = (g.standard_normal((L, Hq * D)).astype(np.float32) for _ in range(3))
+    q = q.reshape(L, Hq, D)
+    q[:, :, 3] = np.abs(q[:, :, 3]) + 0.5                        # times the infinite feature: minus infinity
+    q = q.reshape(L, Hq * D)
+    alive = np.ones(L, bool)
+    for a, b in dead:
+        alive[a:b] = False
+        k[a:b, 3::D] = value
+    # the same softmax in 64 bits over the other keys, of the operands as they are rounded to half
+    h = lambda a: o.from_dt(o.to_dt(a, dt).ravel(), dt).reshape(a.shape).astype(np.float16).astype(np.float64)  # noqa: E731
+    kf = np.where(alive[:, None], k, 0.0).astype(np.float32)
+    want = np.empty((L, Hq * D))
+    for hh in range(Hq):
+        sl = slice(hh * D, hh * D + D)
+        sc = h(q[:, sl]) @ h(kf[:, sl]).T / np.sqrt(D)
+        see = np.broadcast_to(alive, (L, L)) & (np.tri(L, dtype=bool) if form == "causal" else True)
+        sc = np.where(see, sc, -np.inf)
+        with np.errstate(invalid="ignore"):
+            p = np.exp(sc - sc.max(1, keepdims=True))
+        want[:, sl] = p @ h(v[:, sl]) / p.sum(1, keepdims=True)
+    rows = see.any(1)                                            # (a causal row that sees dead keys only has no value)
+    q, k, v = (o.to_dt(a, dt).ravel() for a in (q, k, v))
+    if form == "causal":
+        qt, kt, vt = (up(dev, a, DTS[dt], [L, Hq * D]) for a in (q, k, v))
+        out = new(dev, DTS[dt], [L, Hq * D])
+        R = lambda t: ops.Rows(t, 0, Hq * D, L, Hq, D)  # noqa: E731
+        ops.attention_causal(R(qt), R(kt), R(vt), out)
+        got = out.to_numpy().ravel()
+    else:
+        got = run(dev_16, q, k, v, dt, L, Hq, D, Hq * D, dt)
+    got = o.from_dt(got, dt).astype(np.float32).reshape(L, Hq * D)[rows]
+    assert np.isfinite(got).all(), f"{int((~np.isfinite(got)).any(1).sum())} of {rows.sum()} rows are not finite"
+    rel, _ = o.compare(got.ravel(), want[rows].astype(np.float32).ravel())
+    # P in half, the result in dt: 2^-9 of bfloat16 (relative 2-norm 1.7e-3), under 1e-3 of half's weights
+    assert rel < (3e-3 if dt == o.BF16 else 1e-3), f"relative L2 {rel:.2e}"
