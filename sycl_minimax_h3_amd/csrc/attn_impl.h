@@ -62,12 +62,13 @@ __device__ __forceinline__ uint16_t half_bits(float x) {
 // tell the stages apart), which would make a ring's reads of a landed stage wait for the refills issued after it. The
 // caller's wait_vm before each barrier orders these loads; the memory clobber keeps the compiler from moving LDS
 // accesses across them.
-// (m0 is the compiler's reserved register: it holds nothing across these statements)
+// (m0 is the compiler's reserved register: it holds nothing across these statements. A load to LDS must not be the very
+// next instruction after a scalar write of m0, which inside an asm statement nothing but the s_nop sees to.)
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void attn_dma16(const void* g, const void* lds_dst) {
     const uint32_t m = (uint32_t) (uintptr_t) lds_dst;
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(m) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(m) : "memory", "m0");
 }
 // the same from a wave-uniform base and a 32-bit lane offset; N = 2: a second load 1024 bytes further in both places (the
 // instruction's offset counts for the LDS address too)

@@ -165,3 +165,12 @@ def test_ops_layer_checks_shapes(api):
         ops.Int8Linear(x, w).forward(x, x)
     with pytest.raises(Error, match="twice"):
         ops.swiglu(x, x)
+
+
+def test_scalar_writes_of_m0_are_waited_for():
+    """An inline-asm load to LDS takes its address from m0, and gfx9 needs one instruction between a scalar write of m0 and
+    such a load; the compiler does not look inside asm statements, so each one that writes m0 goes on with an s_nop."""
+    src = os.path.join(ROOT, "sycl_minimax_h3_amd", "csrc")
+    text = "".join(open(os.path.join(src, f)).read() for f in sorted(os.listdir(src)))
+    after = re.findall(r"s_mov_b32 m0, %\d\\n\\t(\w+)", text)
+    assert len(after) >= 4 and len(after) == text.count("s_mov_b32 m0") and set(after) == {"s_nop"}, after
