@@ -41,6 +41,10 @@ constexpr int kAttnRows = 64;            // the reference's scale block (kSageBl
 constexpr int kAttnQBlock = 128;         // queries of a block
 constexpr int kAttnVT = 32;              // keys of a block of the prepared v^T, and of a key tile of the wide kernel
 constexpr int kAttnMaxD = 256;           // the largest head: heads of D features run in kernels of 64, 128 or 256
+// The softmax's reference m before any score has set it: below every score of half operands (at least -2^40 in base 2), and
+// finite, so that tiles of nothing but scores of -infinity (an infinite k's) weigh nothing: 2^(-inf - m) = 0, where m = -inf
+// would give NaN, and a tile's m = kAttnUnset counts for nothing in the merges (2^(kAttnUnset - M) = 0).
+constexpr float kAttnUnset = -3.0e38f;
 // the kernel head size of a head of D features (D <= kAttnMaxD)
 inline int attn_dk(int64_t D) { return D <= 64 ? 64 : D <= 128 ? 128 : 256; }
 
@@ -574,7 +578,7 @@ __global__ __launch_bounds__(256 * KS, KS == 2 ? 2 : DK == 256 ? 1 : 3) void att
     v16f_a o[NDT];
 #pragma unroll
     for (int i = 0; i < NDT; ++i) o[i] = (v16f_a) 0.0f;
-    float m = -INFINITY, l = 0.0f;
+    float m = kAttnUnset, l = 0.0f;
     float ks_cur = SAGE ? P.ks[g * nbp] : 0.0f;               // SAGE: k's scale of the tile being computed
 
     // one 64-key tile; TAIL: the last tile, which holds keys past S
@@ -638,17 +642,14 @@ __global__ __launch_bounds__(256 * KS, KS == 2 ? 2 : DK == 256 ? 1 : 3) void att
         if (__any(mx > m + 8.0f)) {
             asm volatile("" ::: "memory");
             const float mn = fmaxf(m, mx);
-            // (a lane may have seen no live score yet, m = mn = -infinity)
-            const float alpha = m == mn ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+            const float alpha = __builtin_amdgcn_exp2f(m - mn);
             m = mn;
             l = l * alpha;
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt) o[dt] = o[dt] * alpha;
         }
-        // (scores of -infinity, an infinite k's, weigh nothing; before any other score m is still -infinity itself)
-        const float ref = m == -INFINITY ? 0.0f : m;
 #pragma unroll
-        for (int i = 0; i < 32; ++i) x[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[i], f, -ref));
+        for (int i = 0; i < 32; ++i) x[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[i], f, -m));
         if constexpr (TAIL) {
 #pragma unroll
             for (int i = 0; i < 32; ++i)
@@ -950,7 +951,7 @@ __global__ __launch_bounds__(256, 2) void attn_pl_kernel(AttnArgs P) {
     for (int gq = 0; gq < NG; ++gq)
 #pragma unroll
         for (int i = 0; i < NDT; ++i) o[gq][i] = (v16f_a) 0.0f;
-    float m[NG] = {-INFINITY, -INFINITY}, l[NG] = {0.0f, 0.0f};
+    float m[NG] = {kAttnUnset, kAttnUnset}, l[NG] = {0.0f, 0.0f};
     typedef typename std::conditional<SAGE, v16i_a, v16f_a>::type score_t;
     float ks_next = SAGE ? ksc[t0 / 2] : 0.0f;
 
@@ -999,8 +1000,8 @@ __global__ __launch_bounds__(256, 2) void attn_pl_kernel(AttnArgs P) {
             // The weights p = 2^(score f - m) rounded to half, packed as the P v products take them (chunk s: registers
             // 8 s .. 8 s + 7), and their sum over this lane's keys. SAGE: score f - m = x f - (kScoreBias f + m), with
             // one rounding of the offset (relative 2^-24 of kScoreBias f, far below half's rounding of p).
-            auto weights = [&](float ref) {
-                const float c = SAGE ? __builtin_fmaf(kScoreBias, f, ref) : ref;
+            auto weights = [&]() {
+                const float c = SAGE ? __builtin_fmaf(kScoreBias, f, m[gq]) : m[gq];
                 float ls[2];
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
@@ -1026,7 +1027,7 @@ __global__ __launch_bounds__(256, 2) void attn_pl_kernel(AttnArgs P) {
             // 16 above m, or m not yet set) rounds to infinity and makes the lane's sum infinite. Only then the tile's
             // max: m moves when it passes m by more than 8 (as in attn_kernel), O and l are rescaled and the weights
             // computed again (each at most 1 then). O / l does not depend on m.
-            float lt = weights(m[gq]);
+            float lt = weights();
             if (__any(!(lt <= 3.0e38f))) {
                 asm volatile("" ::: "memory");
                 float mt[8];
@@ -1048,9 +1049,7 @@ __global__ __launch_bounds__(256, 2) void attn_pl_kernel(AttnArgs P) {
 #pragma unroll
                     for (int dt = 0; dt < NDT; ++dt) o[gq][dt] = o[gq][dt] * alpha;
                 }
-                // (a tile of scores that are all -infinity, an infinite k's, before any other: they weigh nothing, and m
-                // stays unset)
-                lt = weights(m[gq] == -INFINITY ? 0.0f : m[gq]);
+                lt = weights();
             }
             l[gq] = l[gq] + lt;
             // slice gq's fragments of V^T, into the registers this group's scores leave
