@@ -74,6 +74,51 @@ static void prep(Ctx* c, const void* q, const void* k, const void* v, int64_t S,
 // 61.7 -> 57.7; but 64 heads 600 tokens 23.7 -> 24.7, 2048 tokens 94.5 -> 103 (the blocks fill the device: there two blocks of
 // one group a CU run without a common barrier), and 100 tokens 11.3 -> 12.4 (two tiles: nothing to share out)
 static bool attn_causal_groups(int64_t L, int64_t Hq, int cus) { return L >= 512 && 8 * Hq <= cus; }
+// Which of the wide kernel's n blocks of T key tiles run whole (the first `full`), and into how many blocks of `ts`
+// consecutive tiles each of the others is split (`ns`, at most max_ns; 1: none): the least estimated time, in key tiles of a
+// block that has its CU to itself. Two blocks that share a CU take 1.5 a tile each; a block's start and end cost 5 (1.7 where
+// it is alone); a split costs the merge's launch (7) and every part 0.045 for its partial sums, 130 KiB written and read.
+// Candidates: whole multiples of one or two blocks a CU stay whole, or none (at most two blocks a CU in all). After a round
+// of two blocks a CU, the 16-bit form's next blocks do not spread one a CU: a last round of at most one a CU takes 1.2 there,
+// and a whole block a CU with parts beside it is left to the first round. Parts are bounded by four a CU (133 MiB of scratch
+// on 256 CUs). All choices timed at 1 .. 64 heads, 33 .. 16896 tokens: this takes the fastest, or one within 3 % of it, in 257 of 267
+// cases, and the worst is 10 % off. Splitting whenever a last round filled at most half of two blocks a CU, into
+// as many parts as fitted, lost where a part was short (56 heads: 64 tokens 21.7 -> 14.5 us, 137 tokens 31.7 -> 17.8, 600
+// tokens 52.0 -> 38.7, 1000 tokens 69.9 -> 53.8) and left 257 .. 511 blocks whole (int8 form, 8300 tokens: 8 heads 375 -> 280
+// us, 40 heads 1178 -> 1074; 16896 tokens 4 heads 749 -> 530).
+struct AttnSplit { int64_t full; int ns, ts; };
+static double attn_split_time(int64_t blocks, int64_t T, int64_t cus, double late) {
+    const int64_t rounds = blocks / (2 * cus), rem = blocks % (2 * cus);
+    return (double) rounds * (1.5 * (double) T + 5.0) +
+           (rem == 0 ? 0.0 : rem <= cus ? (rounds ? late : 1.0) * (double) T + 1.7 : 1.5 * (double) T + 5.0);
+}
+static AttnSplit attn_split_plan(int64_t n, int64_t T, int64_t cus, int64_t max_ns, bool sage) {
+    const double late = sage ? 1.0 : 1.2;
+    AttnSplit best{n, 1, 0};
+    double least = attn_split_time(n, T, cus, late);
+    const int64_t fulls[3] = {0, n / cus * cus, n / (2 * cus) * (2 * cus)};
+    for (const int64_t full : fulls) {
+        const int64_t rest = n - full;
+        const bool beside = full % (2 * cus) != 0;             // a whole block a CU, the parts in their CUs' second places
+        if (rest == 0 || rest > 2 * cus || (beside && full > cus && !sage)) continue;
+        for (int64_t want = 2; want <= max_ns && want <= T && rest * want <= 4 * cus; ++want) {
+            const int64_t ts = (T + want - 1) / want, parts = rest * want;
+            if ((T + ts - 1) / ts != want) continue;           // (a smaller count has the same longest part)
+            double t = attn_split_time(full / (2 * cus) * (2 * cus), T, cus, late) + 7.0 + 0.045 * (double) parts;
+            if (beside) {
+                // u tiles beside the whole block, the rest of the longer of the two alone
+                const double u = (double) ((parts + cus - 1) / cus) * ((double) ts + 5.0 / 1.5), w = (double) T;
+                t += 1.7 + (u <= w ? 1.5 * u + (w - u) : 1.5 * w + (u - w));
+            } else {
+                // (parts of more than one round start unevenly)
+                t += attn_split_time(parts, ts, cus, late) * (parts > 2 * cus ? 1.06 : 1.0);
+            }
+            if (t < least) { least = t; best = {full, (int) want, (int) ts}; }
+        }
+    }
+    return best;
+}
+
 // one sequence: S query rows of Hq heads (row stride qs_stride) over S key/value rows of Hkv heads (kv_stride);
 // causal: query i sees keys 0 .. i (the 16-bit form, as the reference's causal kernel computes in float)
 static int attention_one(Ctx* c, const char* fn, const void* q, const void* k, const void* v, int dt, int64_t S, int64_t Hq,
@@ -123,20 +168,16 @@ static int attention_one(Ctx* c, const char* fn, const void* q, const void* k, c
     P.q_dt = dt;
     const int64_t nblocks = Hq * P.nqb;
     P.nfull = nblocks; P.nsplit = 1; P.ts = 0; P.po = nullptr; P.pml = nullptr;
-    // the wide kernel's last round: when it would fill at most half the device (two blocks a CU), its blocks each become up to
-    // c->attn_split blocks of consecutive key tiles, whose results attn_merge_kernel combines
+    // the wide kernel's blocks that are split along the keys (their results combined by attn_merge_kernel)
     int64_t tail = 0;
     if (pp) {
-        const int64_t slots = 2 * (int64_t) c->cus, T = (S + kAttnVT - 1) / kAttnVT, last = nblocks % slots;
-        const int64_t want = std::min<int64_t>({(int64_t) c->attn_split, last ? slots / last : 1, T});
-        if (last > 0 && 2 * last <= slots && want > 1) {
-            const int64_t ts = (T + want - 1) / want, ns = (T + ts - 1) / ts;
-            // (no room for the partial sums under the memory cap: the last round runs unsplit)
-            if (ns > 1 && (P.po = c->scratch<float>(Ctx::ATT_PART, (size_t) (last * ns * kAttnPPQ * (128 + 2))))) {
-                P.pml = P.po + last * ns * kAttnPPQ * 128;
-                tail = last;
-                P.nfull = nblocks - last; P.nsplit = (int) ns; P.ts = (int) ts;
-            }
+        const AttnSplit sp = attn_split_plan(nblocks, (S + kAttnVT - 1) / kAttnVT, c->cus, c->attn_split, sage);
+        const int64_t last = nblocks - sp.full;
+        // (no room for the partial sums under the memory cap: every block runs whole)
+        if (sp.ns > 1 && (P.po = c->scratch<float>(Ctx::ATT_PART, (size_t) (last * sp.ns * kAttnPPQ * (128 + 2))))) {
+            P.pml = P.po + last * sp.ns * kAttnPPQ * 128;
+            tail = last;
+            P.nfull = sp.full; P.nsplit = sp.ns; P.ts = sp.ts;
         }
     }
     const unsigned grid = (unsigned) (P.nfull + tail * P.nsplit);

@@ -446,7 +446,7 @@ struct AttnArgs {
     int nqb;                  // query blocks per head (of 128 queries, or 256 in the wide kernel)
     int kvdiv;                // query heads per key/value head: head h reads k and v of head h / kvdiv
     int64_t Spk;              // rows of the prepared k and v^T (Sp unless they come from another sequence)
-    // the wide kernel's split of the last round: blocks [nfull, nfull + tail * nsplit) each take key tiles
+    // the wide kernel's split blocks: blocks [nfull, nfull + tail * nsplit) each take key tiles
     // [s ts, s ts + ts) of query block nfull + (b - nfull) / nsplit (s = (b - nfull) % nsplit) and leave O, m and l
     // in po / pml for attn_merge_kernel; nfull = the grid and nsplit = 1 when nothing is split
     int64_t nfull;
@@ -790,7 +790,7 @@ constexpr int kScoreBiasBits = 0x4B400000;
 // inside tile t's step, every wavefront issuing its share of the direct loads, which it waits for before the barrier that
 // publishes them (the one inside the step of the tile before). The ring's loads are inline asm (attn_dma16s), and the
 // int8 score products start from kScoreBias's bits: see the helpers above.
-// A block of a split last round (AttnArgs::nfull) walks only its range of key tiles, counted from its first, and
+// A split block (AttnArgs::nfull) walks only its range of key tiles, counted from its first, and
 // leaves O, m and l to attn_merge_kernel.
 template <bool SAGE, int NS>
 __global__ __launch_bounds__(256, 2) void attn_pl_kernel(AttnArgs P) {
@@ -810,7 +810,7 @@ __global__ __launch_bounds__(256, 2) void attn_pl_kernel(AttnArgs P) {
     // heads at a time, which then share K and V^T in its L2)
     // (32-bit block arithmetic: the host keeps the grid below 2^31; 64-bit divisions here delayed every block's start)
     int b = (int) blockIdx.x;
-    // a block of the split last round: its query block and its range of key tiles (slot: its partial sums)
+    // a split block: its query block and its range of key tiles (slot: its partial sums)
     int slot = -1, t0 = 0;
     const int nfull = (int) P.nfull, Tall = (int) ((P.S + kAttnVT - 1) / kAttnVT);
     int T = Tall;

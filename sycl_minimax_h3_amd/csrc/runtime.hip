@@ -167,8 +167,7 @@ static void init(Ctx& c) {
     // H3S_SAGE_MIN_S sets the shortest sequence that takes the int8 (SageAttention) form
     if (const char* e = std::getenv("H3S_ATTN")) c.sage_want = std::strcmp(e, "onednn") != 0;
     if (const char* e = std::getenv("H3S_SAGE_MIN_S")) c.sage_min_s = std::max<int64_t>(0, std::atoll(e));
-    // the pipelined attention kernel: a last round of blocks that fills at most half the CUs is split into up to this
-    // many key ranges a block (1: never)
+    // the wide attention kernel: the most key ranges that it splits a block into (1: never; attn_split_plan)
     if (const char* e = std::getenv("H3S_ATTN_SPLIT")) c.attn_split = std::max(1, std::min(64, std::atoi(e)));
     // the row quantizer's layout: one wavefront a row from this many rows on (four wavefronts a row below)
     if (const char* e = std::getenv("H3S_QUANT_WAVE_MIN_ROWS")) c.quant_wave_min = std::max<int64_t>(0, std::atoll(e));

@@ -166,10 +166,10 @@ def test_attention_kmean(request, blocks, dt, S, H, D):
 
 @pytest.fixture(scope="module")
 def dev_split():
-    """Contexts for the pipelined kernel's split of a short last round, per form: no split (H3S_ATTN_SPLIT=1), the
-    default, and the default with grids sized for 16 or 12 compute units (H3S_CUS), so that a few hundred tokens
-    make full rounds and a split last one (at 12, full blocks that the XCD renumbering leaves in order)."""
-    modes = {"none": {"H3S_ATTN_SPLIT": "1"}, "default": {}, "cus16": {"H3S_CUS": "16"}, "cus12": {"H3S_CUS": "12"}}
+    """Contexts for the wide kernel's split along the keys, per form: no split (H3S_ATTN_SPLIT=1), the default, and the
+    default with grids sized for 16 or 6 compute units (H3S_CUS), so that a few hundred tokens make whole rounds and
+    a split last one (at 6, whole blocks that the XCD renumbering leaves in order)."""
+    modes = {"none": {"H3S_ATTN_SPLIT": "1"}, "default": {}, "cus16": {"H3S_CUS": "16"}, "cus6": {"H3S_CUS": "6"}}
     ds = {}
     for sage in (True, False):
         form = {"H3S_SAGE_MIN_S": "0"} if sage else {"H3S_ATTN": "onednn"}
@@ -181,20 +181,28 @@ def dev_split():
 
 
 @pytest.mark.parametrize("sage", [True, False])
-@pytest.mark.parametrize("mode", ["none", "default", "cus16", "cus12"])
+@pytest.mark.parametrize("mode", ["none", "default", "cus16", "cus6"])
 @pytest.mark.parametrize("S,H", [(64, 1), (777, 3), (2000, 5)])
 def test_attention_split_last_round(dev_split, sage, mode, S, H):
-    """Heads of 128 features (the pipelined kernel). The grids: 64 tokens, one block of one key tile (never split);
-    777 tokens x 3 heads, 12 blocks of 13 tiles (split 7 ways on 256 CUs, not at all on 16 or 12); 2000 x 5, 40 blocks
-    of 32 tiles (6 ways on 256 CUs; on 16, 32 full blocks and 8 split in 2; on 12, 36 full blocks and 4 split in
-    3). The split blocks' partial sums are merged by attn_merge_kernel."""
+    """Heads of 128 features (the wide kernel). The grids (attn_split_plan): 64 tokens, one block of two key tiles (never
+    split); 777 tokens x 3 heads, 12 blocks of 25 tiles (on 256 CUs in 5 parts each, else whole); 2000 x 5, 40 blocks of
+    63 tiles (on 256 CUs in 6 parts each; on 16, 32 whole blocks and 8 in 4; on 6, 36 whole blocks and 4 in 3). The
+    parts' sums are merged by attn_merge_kernel."""
     D = 128
     stride = H * D
     q, k, v = qkv(90 + S, S, H, D, o.BF16, stride)
     want = o.attention(q, k, v, o.BF16, S, H, D, stride, out_dt=o.BF16, sage=sage)
     want = want[0] if sage else want
-    got = run(dev_split[(sage, mode)], q, k, v, o.BF16, S, H, D, stride, o.BF16)
+    d = dev_split[(sage, mode)]
+    got = run(d, q, k, v, o.BF16, S, H, D, stride, o.BF16)
     check(got, want, o.BF16, f"{'int8' if sage else '16-bit'} {mode} S={S} H={H}")
+    t, out = new(d, "BF16", [S, stride]), new(d, "BF16", [S, stride])
+    R = ops.Rows(t, 0, stride, S, H, D)
+    grids = {n.split("<")[0]: b for n, b, _ in launches(d, lambda: ops.attention(R, R, R, out))}
+    whole = H * -(-S // 256)
+    parts = {("default", 777): (0, 5), ("default", 2000): (0, 6), ("cus16", 2000): (32, 4), ("cus6", 2000): (36, 3)}.get((mode, S))
+    assert grids["attn_pl_kernel"] == (parts[0] + (whole - parts[0]) * parts[1] if parts else whole), grids
+    assert ("attn_merge_kernel" in grids) == bool(parts), grids
 
 
 @pytest.mark.parametrize("sage", [True, False])
