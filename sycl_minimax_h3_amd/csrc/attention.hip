@@ -44,7 +44,7 @@ static void prep(Ctx* c, const void* q, const void* k, const void* v, int64_t S,
 #define H3_KV(SG, DD) attn_kv_prep_vec_kernel<DT, SG, DD><<<2 * kvblocks, 256, 0, c->stream>>>(k, v, S, Sp, kv_stride, mean, ak, sc, av)
         if (!vec) {
             qk(k, kv_stride, kvblocks, mean, ak, sc);
-            attn_v_prep_kernel<DT><<<kvblocks, 256, 0, c->stream>>>(v, S, Sp, D, DK, kv_stride, av);
+            attn_v_prep_kernel<DT><<<kvblocks, 256, 0, c->stream>>>(v, S, Sp, D, __builtin_ctz((unsigned) DK), kv_stride, av);
         } else if (sage) {
             if (D == 256) H3_KV(true, 256);
             else if (D == 128) H3_KV(true, 128);
