@@ -9,21 +9,27 @@ namespace h3 {
 
 // out[ci][(r m + mi) C + i] = b[o] + sum_k fl(w[o, k] t[r, k]), o = mi 6 C + ci C + i: the sum in k order from -0.0
 // in float32 (dit.rs:163-170, Rust's f32 Sum), one multiply and one add a term (no fused multiply-add). Bound by the
-// read of w. A wavefront takes 64 consecutive o and NR timestep rows at once (w is read once for them); a tile of 64 o
+// read of w. A wavefront takes 64 consecutive o and NR timestep rows at once (w is read once for them; blockIdx.y counts the
+// groups of NR rows, the last one's missing rows repeating the last row, not stored); a tile of 64 o
 // x 32 k goes through registers to LDS in 16-byte pieces that cover whole 128-byte lines, two tiles in flight while
 // the one before is summed, and each lane runs its own o's NR sums (t[r, k] is a scalar operand). The LDS rows are 36
 // floats apart, so 16 lanes' 16-byte reads touch every bank once. VEC = 1 (rows that are not whole 16-byte pieces)
 // loads single floats the same way. 96768 x 256 floats with 2 timesteps, and the
 // rotations of 2159 tokens: 185.6 -> 22.6 us (the tables alone were 152, 64 dependent row loads a tile and w read once a
-// timestep; the 101 MB take 20 us at the rate of a large copy).
+// timestep; the 101 MB take 20 us at the rate of a large copy). All groups in one launch: with few outputs and many timesteps
+// a launch a group leaves the device idle (R = 1000, 384 x 256 floats: 3251 us, 99 with one launch of a row a block, 17.6 here).
 constexpr int kTabK = 32, kTabStride = kTabK + 4;
 template <int NR, int VEC>
 __global__ __launch_bounds__(64) void adaln_tables_kernel(const float* __restrict__ w, const float* __restrict__ b,
-                                                          const float* __restrict__ t, int64_t R, int64_t r0, int64_t td,
-                                                          int64_t m, int64_t C, float* __restrict__ out) {
+                                                          const float* __restrict__ t, int64_t R, int64_t td, int64_t m,
+                                                          int64_t C, float* __restrict__ out) {
     constexpr int LPR = kTabK / VEC, RPL = 64 / LPR, NL = 64 / RPL;   // lanes a row, rows a load, loads a tile
     typedef float fvec __attribute__((ext_vector_type(VEC)));
-    __shared__ float tile[64 * kTabStride];
+    __shared__ __attribute__((aligned(16))) float tile[64 * kTabStride];
+    const int64_t r0 = (int64_t) blockIdx.y * NR;
+    int64_t row[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) row[r] = r0 + r < R ? r0 + r : R - 1;
     const int lane = threadIdx.x, lr = lane / LPR, lk = lane % LPR * VEC;
     const int64_t nout = 6 * m * C, o0 = (int64_t) blockIdx.x * 64, o = o0 + lane;
     float sum[NR];
@@ -46,14 +52,14 @@ __global__ __launch_bounds__(64) void adaln_tables_kernel(const float* __restric
         fetch(f, k0 + 2 * kTabK);
         lds_barrier();
         const float* mine = &tile[lane * kTabStride];
-        const float* tk = t + r0 * td + k0;
+        const float* tk = t + k0;
         if (k0 + kTabK <= td) {
 #pragma unroll
             for (int k = 0; k < kTabK; k += 4) {
                 const float4 v = *reinterpret_cast<const float4*>(mine + k);
 #pragma unroll
                 for (int r = 0; r < NR; ++r) {
-                    const float* tr = tk + r * td + k;
+                    const float* tr = tk + row[r] * td + k;
                     sum[r] = sum[r] + v.x * tr[0];
                     sum[r] = sum[r] + v.y * tr[1];
                     sum[r] = sum[r] + v.z * tr[2];
@@ -64,7 +70,7 @@ __global__ __launch_bounds__(64) void adaln_tables_kernel(const float* __restric
             for (int k = 0; k < td - k0; ++k) {
                 const float v = mine[k];
 #pragma unroll
-                for (int r = 0; r < NR; ++r) sum[r] = sum[r] + v * tk[r * td + k];
+                for (int r = 0; r < NR; ++r) sum[r] = sum[r] + v * tk[row[r] * td + k];
             }
         }
         lds_barrier();
@@ -80,18 +86,19 @@ __global__ __launch_bounds__(64) void adaln_tables_kernel(const float* __restric
     float* p = out + ci * R * m * C + mi * C + i;
     const float bo = b[o];
 #pragma unroll
-    for (int r = 0; r < NR; ++r) p[(r0 + r) * m * C] = bo + sum[r];
+    for (int r = 0; r < NR; ++r)
+        if (r0 + r < R) p[(r0 + r) * m * C] = bo + sum[r];
 }
 
 template <int VEC>
 static void adaln_tables(Ctx* c, const float* w, const float* b, const float* t, int64_t R, int64_t td, int64_t m, int64_t C,
                          float* out) {
-    const unsigned blocks = (unsigned) ((6 * m * C + 63) / 64);
-    int64_t r = 0;
-    for (; R - r >= 4; r += 4) adaln_tables_kernel<4, VEC><<<blocks, 64, 0, c->stream>>>(w, b, t, R, r, td, m, C, out);
-    if (R - r == 3) adaln_tables_kernel<3, VEC><<<blocks, 64, 0, c->stream>>>(w, b, t, R, r, td, m, C, out);
-    else if (R - r == 2) adaln_tables_kernel<2, VEC><<<blocks, 64, 0, c->stream>>>(w, b, t, R, r, td, m, C, out);
-    else if (R - r == 1) adaln_tables_kernel<1, VEC><<<blocks, 64, 0, c->stream>>>(w, b, t, R, r, td, m, C, out);
+    const int64_t nr = R < 4 ? R : 4;
+    const dim3 grid((unsigned) ((6 * m * C + 63) / 64), (unsigned) ((R + nr - 1) / nr));
+    if (nr == 4) adaln_tables_kernel<4, VEC><<<grid, 64, 0, c->stream>>>(w, b, t, R, td, m, C, out);
+    else if (nr == 3) adaln_tables_kernel<3, VEC><<<grid, 64, 0, c->stream>>>(w, b, t, R, td, m, C, out);
+    else if (nr == 2) adaln_tables_kernel<2, VEC><<<grid, 64, 0, c->stream>>>(w, b, t, R, td, m, C, out);
+    else adaln_tables_kernel<1, VEC><<<grid, 64, 0, c->stream>>>(w, b, t, R, td, m, C, out);
 }
 
 // cs[s][a n + f] = (cos x, sin x), x = fl((float) pos[s, a] * inv_freq[f]) (dit.rs:190-203); cos and sin of the float
@@ -118,6 +125,7 @@ H3S_EXPORT int h3s_adaln_tables(void* ctx, const float* w, const float* b, const
     const char* fn = "h3s_adaln_tables";
     if (R <= 0 || t_dim <= 0 || m <= 0 || C <= 0) return 0;
     if (!w || !b || !t_emb || !out) return fail(std::string(fn) + ": w, b, t_emb and out are required");
+    // (a bound of the interface, since a timestep row was a block of the grid's second dimension)
     if (R > 65535) return fail(std::string(fn) + ": at most 65535 timestep rows");
     Ctx* c = ctx_of(ctx, fn);
     if (!c) return -1;

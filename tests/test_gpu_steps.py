@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as o
-from helpers import new, up
+from helpers import launches, new, up
 from sycl_minimax_h3_amd import DType, Error, ops
 from sycl_minimax_h3_amd.layout import Request, place, plan, step_rows
 
@@ -39,6 +39,16 @@ def test_adaln_tables_tiles(dev, R, td, m, C):
     """the edges of the kernel's tiles: one, two, three and more tiles of 32 columns, a last tile cut short, rows of
     whole 16-byte pieces and not, a last group of fewer than 64 outputs, and one to four timesteps a pass"""
     test_adaln_tables(dev, R, td, m, C)
+
+
+@pytest.mark.parametrize("R,td,m,C", [(1, 64, 1, 64), (4, 256, 1, 64), (7, 32, 2, 16), (1001, 36, 1, 5)])
+def test_adaln_tables_one_launch(dev, R, td, m, C):
+    """any number of timesteps in one launch, and their values"""
+    test_adaln_tables(dev, R, td, m, C)
+    w, b, t = new(dev, "F32", [6 * m * C, td]), new(dev, "F32", [6 * m * C]), new(dev, "F32", [R, td])
+    out = new(dev, "F32", [6, R * m, C])
+    got = launches(dev, lambda: ops.adaln_tables(w, b, t, m, out))
+    assert len(got) == 1, got
 
 
 def test_rotations_wide(dev):
