@@ -589,7 +589,7 @@ inline void gemm_plan_split(int64_t tiles, int64_t nk, int cus, int* main_tiles,
 // 5376 -> 14336, cold weights: 640 rows 123 -> 112, 768 128 -> 121, 520 115 -> 117.) A split launch's parts
 // are written and read at about 0.1 us a part of 256 live rows. Short products (below 32 steps) keep 256 rows: there the
 // epilogue, not the steps, is the time.
-struct GemmPlan { int wi, main_tiles, split; };
+struct GemmPlan { int wi, main_tiles, split; double us; };   // (us: the steps' estimate)
 inline double gemm_round_us(int64_t tiles, int wi, int cus) {
     const double full = wi == 4 ? 1.75 : wi == 3 ? 1.33 : 1.0, least = wi == 4 ? 1.05 : wi == 3 ? 0.95 : 0.82;
     const double f = (double) (tiles % cus) / cus;
@@ -597,21 +597,22 @@ inline double gemm_round_us(int64_t tiles, int wi, int cus) {
 }
 inline GemmPlan gemm_plan(int64_t M, int64_t N, int64_t nk, int cus, bool may_split) {
     const int64_t tn = (N + kGemmBN - 1) / kGemmBN, tm = (M + kGemmBM - 1) / kGemmBM, tiles = tm * tn;
-    GemmPlan p{4, (int) tiles, 1};
+    GemmPlan p{4, (int) tiles, 1, 0.0};
     if (may_split) gemm_plan_split(tiles, nk, cus, &p.main_tiles, &p.split);
-    if (nk < 32) return p;
     double us = gemm_round_us(p.main_tiles, 4, cus) * (double) nk;
     if (p.split > 1) {
         const int64_t parts = (tiles - p.main_tiles) * p.split;
         us += gemm_round_us(parts, 4, cus) * (double) ((nk + p.split - 1) / p.split) + 3.0 +
               0.1 * (double) parts * (double) M / (double) (tm * kGemmBM);
     }
+    p.us = us;
+    if (nk < 32) return p;
     us *= 0.97;
     for (int wi = 3; wi >= 2; --wi) {
         const int64_t t = (M + 64 * wi - 1) / (64 * wi) * tn;
         if (t > 0x7fffffff) break;
         const double u = gemm_round_us(t, wi, cus) * (double) nk;
-        if (u < us) { us = u; p = {wi, (int) t, 1}; }
+        if (u < us) { us = u; p = {wi, (int) t, 1, u}; }
     }
     return p;
 }

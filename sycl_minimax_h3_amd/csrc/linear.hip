@@ -107,7 +107,7 @@ static void merge_f16(Ctx* c, const GemmArgs& P, unsigned mgrid) {
 static int linear_mfma(Ctx* c, const char* fn, const void* x, int dt, int64_t M, int64_t K, const void* w, int64_t N,
                        const float* bias, void* out, int out_dt, bool acc) {
     const int64_t tn = (N + kGemmBN - 1) / kGemmBN, kb = 2 * K;
-    GemmPlan plan{4, 0, 1};
+    GemmPlan plan{4, 0, 1, 0.0};
     if (acc) {
         const int64_t tiles = (M + kGemmBM - 1) / kGemmBM * tn;
         plan.main_tiles = (int) tiles;
@@ -161,9 +161,9 @@ static void skinny_mt(Ctx* c, const SkinnyArgs& P, int mt, int nt) {
 // 128, the choice is within 10 % of the fastest of all tiles and parts): a CU takes about 2.4 ns a row and step and at
 // least 250 ns a step, the blocks run in rounds of one a CU, memory gives about 5 TB/s (7 for what the 256 MB cache beside
 // it may hold), and parts cost their float32 sums written and read once and the merge's launch.
-struct SkinnyPlan { int mt, nt, parts; double us; };
+struct SkinnyPlan { int mt, nt, parts; int64_t blocks, rows; double us; };
 static SkinnyPlan skinny_plan(int64_t S, int64_t L, int64_t nk, int cus) {
-    SkinnyPlan best{0, 0, 0, 1e300};
+    SkinnyPlan best{0, 0, 0, 0, 0, 1e300};
     const int64_t ts = (S + 255) / 256;
     const int mt = (int) ((S + 64 * ts - 1) / (64 * ts));
     const int64_t rows = (S + ts - 1) / ts;
@@ -175,24 +175,64 @@ static SkinnyPlan skinny_plan(int64_t S, int64_t L, int64_t nk, int cus) {
                                std::max(0.25, 0.0024 * (double) (rows + 64 * nt));
             const double bytes = (double) (S + L) * (double) nk * kGemmBK, floor = bytes / (bytes > 256e6 ? 5e6 : 7e6);
             const double us = std::max(run, floor) + (parts > 1 ? 2.0 + (double) parts * (double) S * (double) L * 8 / 3.5e6 : 0.0);
-            if (us < best.us) best = {mt, nt, parts, us};
+            if (us < best.us) best = {mt, nt, parts, blocks, rows, us};
         }
     return best;
 }
+// Whether gemm_impl.h's tiles take a product that skinny_plan has planned (p) after all: not where its tiles are split in
+// parts; where it takes several rounds of more than 64 rows, unless their loads alone take the time (an out of few columns: up
+// to 16 steps); and else by the two whole times in microseconds. Here: 0.0026 a row and step, a block's end (the groups'
+// exchange, 8-byte stores) 0.76 a 64 x 64 piece and round, 3.8 for the launch. There: gemm_plan's estimate, 3.9 for the
+// launch with the short epilogue of a tile inside out, 0.035 more a live row of a tile cut at out's edge (its stores go
+// element by element), 5.5 with a merge. Operands past the 256 MB cache come at 6.5 TB/s here, by the blocks' share of the
+// CUs, and there at 5, and a step of 256, 192 or 128 rows then takes 1.75, 1.55 or 1.33 however few the blocks. Timed both
+// ways over 1 .. 512 rows against 256 .. 65536 outputs, and 513 .. 47104 against 8 .. 128, of 64 .. 14336 features (bfloat16,
+// 2099 products): the choice is 0.3 % off the faster on average, and within 5 % of it in 97 %. Always here, products of one to
+// four steps and of more outputs than fill one round had lost to the tiles: 512 rows 64 -> 28672 8.5 -> 24.1 us, 512 rows
+// 5376 -> 28672 143 -> 174, 256 rows 64 -> 5376 5.7 -> 7.9.
+static bool skinny_loses(const SkinnyPlan& p, bool swap, int64_t M, int64_t N, int64_t nk, int cus) {
+    if (p.parts > 1) return false;
+    const int64_t round = (int64_t) cus * skinny_per_cu(p.mt, p.nt), rounds = (p.blocks + round - 1) / round;
+    const double bytes = (double) (M + N) * (double) nk * kGemmBK;
+    const bool cached = bytes <= 256e6;
+    const double run = (double) ((p.blocks + cus - 1) / cus * nk) * std::max(0.25, 0.0026 * (double) (p.rows + 64 * p.nt));
+    const double from = cached ? bytes / 7e6 : bytes / (6.5e6 * std::min(1.0, (double) p.blocks / cus));
+    const bool by_loads = p.us <= 1.0001 * bytes / (cached ? 7e6 : 5e6);
+    if (rounds > 1 && p.rows > 64 && (swap ? nk <= 16 : M > 256 || !by_loads)) return true;
+    const GemmPlan g = gemm_plan(M, N, nk, cus, true);
+    const int64_t bm = 64 * g.wi, tm = (M + bm - 1) / bm, tn = (N + kGemmBN - 1) / kGemmBN;
+    double tiles = g.us;
+    if (!cached) {
+        const double step = g.wi == 4 ? 1.75 : g.wi == 3 ? 1.55 : 1.33;
+        double t = (double) ((g.main_tiles + cus - 1) / cus * nk) * step;
+        if (g.split > 1)
+            t += (double) ((nk + g.split - 1) / g.split) * step +
+                 0.1 * (double) ((tm * tn - g.main_tiles) * g.split) * std::min(1.0, (double) M / kGemmBM);
+        tiles = std::max({tiles, t, bytes / 5e6});
+    }
+    int64_t cut = 0;                                             // live rows that cut tiles store one after the other
+    if (g.split == 1) {
+        cut = M % bm * ((tn + cus - 1) / cus);
+        if (N % kGemmBN) cut = std::max(cut, std::min(M, bm) * ((tm + cus - 1) / cus));
+    }
+    const double here = 3.8 + 0.76 * (double) (p.mt * p.nt * rounds) + std::max(run, from);
+    const double there = 3.9 + 0.035 * (double) cut + (g.split > 1 ? 5.5 : 0.0) + tiles;
+    return there < here;
+}
 // h3s_linear with few rows on one side (gemm_skinny.h): at most 512 rows of x, or at most 128 of w. Above, gemm_impl.h's
 // tiles have the rows to fill them (768 rows 5376 -> 5376: 65 against 66 us at the best tile here; 256 rows of w at 16896
-// tokens 95 against 137). 1: not a shape it takes.
+// tokens 95 against 137). 1: not a product it takes.
 static int linear_skinny(Ctx* c, const char* fn, const void* x, int dt, int64_t M, int64_t K, const void* w, int64_t N,
                          const float* bias, void* out, int out_dt) {
     const int64_t kb = 2 * K, nk = (kb + kGemmBK - 1) / kGemmBK;
-    SkinnyPlan p{0, 0, 0, 1e300};
+    SkinnyPlan p{0, 0, 0, 0, 0, 1e300};
     bool swap = false;
     if (M <= 512) p = skinny_plan(M, N, nk, c->cus);
     if (N <= 128) {
         const SkinnyPlan q = skinny_plan(N, M, nk, c->cus);
         if (q.us < p.us) { p = q; swap = true; }
     }
-    if (!p.mt) return 1;
+    if (!p.mt || skinny_loses(p, swap, M, N, nk, c->cus)) return 1;
     const int64_t S = swap ? N : M, L = swap ? M : N;
     const int64_t ts = (S + 64 * p.mt - 1) / (64 * p.mt), tl = (L + 64 * p.nt - 1) / (64 * p.nt);
     if (ts * tl * 64 > 0x7fffffff) return 1;                     // (blocks, and the merge's, within 32 bits)

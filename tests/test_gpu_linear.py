@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as o
-from helpers import assert_bits_equal, assert_close_16, new, up
+from helpers import assert_bits_equal, assert_close_16, launches, new, up
 from sycl_minimax_h3_amd import DType, ops
 
 pytestmark = pytest.mark.gpu
@@ -55,6 +55,21 @@ def test_linear(dev, dt, out_dt, M, K, N, bias):
 @pytest.mark.parametrize("dt,out_dt,bias", [(o.BF16, o.BF16, True), (o.F16, o.F16, False), (o.BF16, o.F32, True)])
 def test_linear_few_rows(dev, dt, out_dt, bias, M, K, N):
     test_linear(dev, dt, out_dt, M, K, N, bias)
+
+
+@pytest.mark.parametrize("few,M,K,N", [(True, 137, 64, 512), (False, 256, 64, 512), (False, 512, 128, 2048), (True, 400, 64, 256),
+                                       (False, 400, 96, 21504), (True, 64, 128, 16384), (True, 512, 2048, 2048), (False, 47104, 64, 96),
+                                       (True, 47104, 64, 32), (True, 513, 64, 128), (False, 513, 64, 129)])
+def test_linear_few_rows_or_tiles(dev, few, M, K, N):
+    """which of the two matrix-core kernels takes a product with few rows on one side (skinny_loses): few steps with whole
+    256 x 256 tiles, or more than a round of blocks, go to the tiles, the others to the few-row kernel"""
+    x, w, b = mats(130, M, K, N, o.BF16)
+    want = o.linear(x, o.BF16, M, K, w, N, b, out_dt=o.BF16)
+    out, layer = new(dev, "BF16", [M, N]), ops.Linear(up(dev, w, "BF16", [N, K]), up(dev, b, "F32", [N]))
+    xt = up(dev, x, "BF16", [M, K])
+    names = [n.split("<")[0] for n, _, _ in launches(dev, lambda: layer.forward(xt, out))]
+    close(out.to_numpy(), want, o.BF16, "linear")
+    assert names[0] == ("gemm_skinny_kernel" if few else "gemm_f16_kernel"), names
 
 
 @pytest.mark.parametrize("M,K,N", [(8300, 128, 64), (700, 1024, 600), (300, 96, 260), (130, 200, 70)])
