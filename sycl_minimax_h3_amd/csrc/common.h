@@ -74,8 +74,10 @@ struct Ctx {
     bool sage_want = true;                 // H3S_ATTN=onednn: false
     int64_t sage_min_s = 8192;             // H3S_SAGE_MIN_S
     int attn_split = 8;                    // H3S_ATTN_SPLIT: most key ranges a block of the wide attention is split into (1: none)
-    int64_t quant_wave_min = 8192;         // H3S_QUANT_WAVE_MIN_ROWS: rows from which the quantizer takes one wavefront a row
-                                           // (some shapes from a fixed share of it: quant_launch)
+    // H3S_QUANT_WAVE_MIN_ROWS: rows from which the quantizer takes one wavefront a row, for every row shape; not set (-1), each
+    // shape has a line of its own
+    int64_t quant_wave_min = -1;
+    int64_t quant_line(int64_t rows) const { return quant_wave_min >= 0 ? quant_wave_min : rows; }
     // H3S_PROFILE (kernels/h3sycl.cpp:117, 228): the int8 linear's time by pass, summed over its row chunks and
     // reported at h3s_destroy; attention's time by phase, reported per call
     bool profile = false;

@@ -1121,13 +1121,12 @@ template <int XDT> int quant_launch(Ctx* c, const char* fn, const QuantArgs& A, 
     if (mode == QUANT_NORM_OUT) f |= ROW_OUTH;
     // the model's widths, one or two wavefronts a row
     if constexpr (XDT != H3S_F32) {
-        // From quant_wave_min (8192) rows; with the checkpoints' rotation from an eighth of it: the pair layout's rotation
-        // takes fewer instructions than the general kernel's, which shows as soon as the launch is longer than its latency
+        // From 8192 rows; with the checkpoints' rotation from 1024: the pair layout's rotation takes fewer instructions than the general kernel's, which shows as soon as the launch is longer than its latency
         // (2159 rows: swiglu 14336 36.0 -> 31.3 us, x 14336 25.8 -> 20.7, norm with
         // tables 22.2 -> 17.2; 1024 rows: 18.7 -> 14.9, 13.5 -> 9.5, 11.5 -> 9.2). Unrotated the two are alike up to 6000
         // rows (7168 features at 2159 rows: 8.5 general, 10.4 here).
         const bool reg256 = A.rot == H3S_ROT_REGULAR && A.group == 256;
-        if (quant_wave_model_takes(A, f) && (A.M >= (reg256 ? c->quant_wave_min / 8 : c->quant_wave_min) || (f & ROW_OUTH))) {
+        if (quant_wave_model_takes(A, f) && (A.M >= c->quant_line(reg256 ? 1024 : 8192) || (f & ROW_OUTH))) {
             const int r = quant_wave_model<XDT>(c, fn, A, f);
             if (r != 1) return r;
         }
@@ -1154,15 +1153,14 @@ template <int XDT> int quant_launch(Ctx* c, const char* fn, const QuantArgs& A, 
     }                                                                                                \
     H3_QUANT_F(CC, RR, ROW_DYN);                                                                     \
     return launched(fn);
-    // rows of 2048 or 4096 features of a 16-bit type with the exact side inputs, and enough of them (the context's
-    // quant_wave_min, 8192) to give every wavefront several rows: one wavefront a row (fewer rows: four wavefronts
-    // share each, which shortens a short launch). The norm without a table row per token needs no persistent blocks and
-    // pays from three eighths of it (4096 features, weight only: 3000 rows 11.3 -> 9.5 us, 4096 rows 14.8 -> 12.7, one
+    // rows of 2048 or 4096 features of a 16-bit type with the exact side inputs, and enough of them (8192) to give every
+    // wavefront several rows: one wavefront a row (fewer rows: four wavefronts share each, which shortens a short launch).
+    // The norm without a table row per token needs no persistent blocks and pays from 3072 (4096 features, weight only: 3000 rows 11.3 -> 9.5 us, 4096 rows 14.8 -> 12.7, one
     // table row 18.9 -> 14.0; 2159 rows 9.0 against 9.2); with a table row per token 4096 rows take 19.9 general, 20.9 here.
     if constexpr (XDT != H3S_F32) {
         if ((f == kQuantNone || f == kQuantW || f == kQuantWTab || f == kQuantWTab32 || f == kQuantRaw) &&
             (A.C == 2048 || A.C == 4096) &&
-            A.M >= (f == kQuantRaw || ((f & ROW_TAB) && A.rows) ? c->quant_wave_min : c->quant_wave_min / 8 * 3)) {
+            A.M >= c->quant_line(f == kQuantRaw || ((f & ROW_TAB) && A.rows) ? 8192 : 3072)) {
             if (A.C == 2048) return quant_wave_launch<XDT, 4>(c, fn, A, f);
             return quant_wave_launch<XDT, 8>(c, fn, A, f);
         }

@@ -169,7 +169,8 @@ static void init(Ctx& c) {
     if (const char* e = std::getenv("H3S_SAGE_MIN_S")) c.sage_min_s = std::max<int64_t>(0, std::atoll(e));
     // the wide attention kernel: the most key ranges that it splits a block into (1: never; attn_split_plan)
     if (const char* e = std::getenv("H3S_ATTN_SPLIT")) c.attn_split = std::max(1, std::min(64, std::atoi(e)));
-    // the row quantizer's layout: one wavefront a row from this many rows on (four wavefronts a row below)
+    // the row quantizer's layout: one wavefront a row from this many rows on (four wavefronts a row below), in place of the
+    // lines that the row shapes have
     if (const char* e = std::getenv("H3S_QUANT_WAVE_MIN_ROWS")) c.quant_wave_min = std::max<int64_t>(0, std::atoll(e));
 }
 

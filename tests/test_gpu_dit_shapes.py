@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as o
-from helpers import assert_bits_equal, codes_close, new, up
+from helpers import assert_bits_equal, codes_close, launches, new, up
 
 pytestmark = pytest.mark.gpu
 
@@ -102,6 +102,40 @@ def test_norm_quant_layout_lines(dev, C, M, tables):
     ops.norm_quant(up(dev, x, "BF16", [M, C]), up(dev, w, "F32", [C]), 1e-5, tb, q, s, rot=rot, group=group)
     assert_bits_equal(s.to_numpy(), want_s, "scales")
     codes_close(q.to_numpy(), want_q, "codes")
+
+
+@pytest.fixture(scope="module")
+def dev_rows5000():
+    """A context told to take the one-wavefront-a-row layouts from 5000 rows (H3S_QUANT_WAVE_MIN_ROWS)."""
+    import os
+    from sycl_minimax_h3_amd import Device
+
+    old = os.environ.get("H3S_QUANT_WAVE_MIN_ROWS")
+    os.environ["H3S_QUANT_WAVE_MIN_ROWS"] = "5000"
+    try:
+        d = Device.open()
+    finally:
+        if old is None:
+            del os.environ["H3S_QUANT_WAVE_MIN_ROWS"]
+        else:
+            os.environ["H3S_QUANT_WAVE_MIN_ROWS"] = old
+    yield d
+    d.close()
+
+
+@pytest.mark.parametrize("M,wave", [(1024, False), (4999, False), (5000, True), (8192, True)])
+@pytest.mark.parametrize("kind,C,rot,group", [("norm", 5376, o.ROT_REGULAR, 256), ("norm", 4096, o.ROT_SYLVESTER, 128), ("raw", 7168, o.ROT_REGULAR, 256),
+                                              ("raw", 2048, o.ROT_NONE, 0), ("swiglu", 8192, o.ROT_REGULAR, 256), ("raw", 7168, o.ROT_NONE, 0)])
+def test_quant_rows_of_the_environment(dev_rows5000, kind, C, rot, group, M, wave):
+    """H3S_QUANT_WAVE_MIN_ROWS is the line for every row shape: four wavefronts a row below it, one layout above"""
+    dev = dev_rows5000
+    x, q, s = new(dev, "BF16", [M, 2 * C if kind == "swiglu" else C]), new(dev, "I8", [M, C]), new(dev, "F32", [M])
+    w = new(dev, "F32", [C])
+    call = {"norm": lambda: ops.norm_quant(x, w, 1e-5, None, q, s, rot=rot, group=group),
+            "raw": lambda: ops.int8_quantize(x, q, s, group),
+            "swiglu": lambda: ops.swiglu_quant(x, q, s, rot=rot, group=group)}[kind]
+    names = [n.split("<")[0] for n, _, _ in launches(dev, call)]
+    assert names == ["quant_wave_kernel" if wave else "quant_kernel"], names
 
 
 @pytest.mark.parametrize("layout", ["four", "wave"])
