@@ -1124,9 +1124,10 @@ template <int XDT> int quant_launch(Ctx* c, const char* fn, const QuantArgs& A, 
         // From 8192 rows; with the checkpoints' rotation from 1024: the pair layout's rotation takes fewer instructions than the general kernel's, which shows as soon as the launch is longer than its latency
         // (2159 rows: swiglu 14336 36.0 -> 31.3 us, x 14336 25.8 -> 20.7, norm with
         // tables 22.2 -> 17.2; 1024 rows: 18.7 -> 14.9, 13.5 -> 9.5, 11.5 -> 9.2). Unrotated the two are alike up to 6000
-        // rows (7168 features at 2159 rows: 8.5 general, 10.4 here).
+        // rows (7168 features at 2159 rows: 8.5 general, 10.4 here). The norm without tables from 2560 (1500 rows 10.4 general,
+        // 10.8 here, 2159 rows 13.6, 14.0, 3071 rows 17.5, 14.5).
         const bool reg256 = A.rot == H3S_ROT_REGULAR && A.group == 256;
-        if (quant_wave_model_takes(A, f) && (A.M >= c->quant_line(reg256 ? 1024 : 8192) || (f & ROW_OUTH))) {
+        if (quant_wave_model_takes(A, f) && (A.M >= c->quant_line(!reg256 ? 8192 : f == kQuantW ? 2560 : 1024) || (f & ROW_OUTH))) {
             const int r = quant_wave_model<XDT>(c, fn, A, f);
             if (r != 1) return r;
         }
@@ -1155,12 +1156,19 @@ template <int XDT> int quant_launch(Ctx* c, const char* fn, const QuantArgs& A, 
     return launched(fn);
     // rows of 2048 or 4096 features of a 16-bit type with the exact side inputs, and enough of them (8192) to give every
     // wavefront several rows: one wavefront a row (fewer rows: four wavefronts share each, which shortens a short launch).
-    // The norm without a table row per token needs no persistent blocks and pays from 3072 (4096 features, weight only: 3000 rows 11.3 -> 9.5 us, 4096 rows 14.8 -> 12.7, one
-    // table row 18.9 -> 14.0; 2159 rows 9.0 against 9.2); with a table row per token 4096 rows take 19.9 general, 20.9 here.
+    // The norm without a table row per token needs no persistent blocks and pays from 3072 (4096 features, weight only: 3000
+    // rows 11.3 -> 9.5 us, 4096 rows 14.8 -> 12.7, one table row 18.9 -> 14.0; 2159 rows 9.0 against 9.2); with a table row per
+    // token 4096 rows take 19.9 general, 20.9 here. The regular rotation, and Sylvester groups other than 128, cost this layout
+    // more: at 4096 features the norm without tables takes longer up to 8192 rows (group 256 at 3072 rows 12.5 general, 14.3
+    // here; group 64 at 6000 rows 19.1, 21.4; Sylvester groups of 64 at 5000 rows 15.7, 16.4), and with a table or 2048 features
+    // the two of the regular rotation cross between 3072 rows (2048 features 9.1, 10.1) and 4096 (12.1, 10.3).
     if constexpr (XDT != H3S_F32) {
+        const bool costly = A.rot == H3S_ROT_REGULAR || (A.rot == H3S_ROT_SYLVESTER && A.group != 128), tab = (f & ROW_TAB) != 0;
+        const int64_t line = f == kQuantRaw || (tab && A.rows) || (costly && A.C == 4096 && !tab) ? 8192
+                             : A.rot == H3S_ROT_REGULAR                                            ? 4096
+                                                                                                   : 3072;
         if ((f == kQuantNone || f == kQuantW || f == kQuantWTab || f == kQuantWTab32 || f == kQuantRaw) &&
-            (A.C == 2048 || A.C == 4096) &&
-            A.M >= c->quant_line(f == kQuantRaw || ((f & ROW_TAB) && A.rows) ? 8192 : 3072)) {
+            (A.C == 2048 || A.C == 4096) && A.M >= c->quant_line(line)) {
             if (A.C == 2048) return quant_wave_launch<XDT, 4>(c, fn, A, f);
             return quant_wave_launch<XDT, 8>(c, fn, A, f);
         }

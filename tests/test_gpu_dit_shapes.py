@@ -104,6 +104,23 @@ def test_norm_quant_layout_lines(dev, C, M, tables):
     codes_close(q.to_numpy(), want_q, "codes")
 
 
+@pytest.mark.parametrize("C,rot,group,tables,line", [(4096, o.ROT_REGULAR, 256, None, 8192), (4096, o.ROT_REGULAR, 64, None, 8192),
+                                                     (4096, o.ROT_REGULAR, 256, "one", 4096), (2048, o.ROT_REGULAR, 64, None, 4096),
+                                                     (2048, o.ROT_REGULAR, 256, "one", 4096), (4096, o.ROT_SYLVESTER, 128, None, 3072),
+                                                     (4096, o.ROT_SYLVESTER, 64, None, 8192), (5376, o.ROT_REGULAR, 256, None, 2560),
+                                                     (2048, o.ROT_NONE, 0, "one", 3072), (4096, o.ROT_NONE, 0, "rows", 8192),
+                                                     (5376, o.ROT_REGULAR, 256, "rows", 1024)])
+def test_norm_quant_default_lines(dev, C, rot, group, tables, line):
+    """the row count from which the default context takes one wavefront a row, by row shape and rotation"""
+    for M in (line - 1, line):
+        x, q, s = new(dev, "BF16", [M, C]), new(dev, "I8", [M, C]), new(dev, "F32", [M])
+        w, tab = new(dev, "F32", [C]), new(dev, "F32", [2, C])
+        rows = up(dev, dit_rows(M), "I32", [M]) if tables == "rows" else None
+        tb = ops.Tables(scale=tab, shift=tab, rows=rows) if tables else None
+        names = [n.split("<")[0] for n, _, _ in launches(dev, lambda: ops.norm_quant(x, w, 1e-5, tb, q, s, rot=rot, group=group))]
+        assert names == ["quant_kernel" if M < line else "quant_wave_kernel"], (M, names)
+
+
 @pytest.fixture(scope="module")
 def dev_rows5000():
     """A context told to take the one-wavefront-a-row layouts from 5000 rows (H3S_QUANT_WAVE_MIN_ROWS)."""
