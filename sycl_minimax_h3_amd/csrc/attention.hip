@@ -29,8 +29,8 @@ static void prep(Ctx* c, const void* q, const void* k, const void* v, int64_t S,
             if (sage) attn_qk_prep_kernel<DT, true><<<blocks, 256, 0, c->stream>>>(src, S, Sp, D, DK, stride, mean, dst, sc);
             else attn_qk_prep_kernel<DT, false><<<blocks, 256, 0, c->stream>>>(src, S, Sp, D, DK, stride, mean, dst, sc);
         } else if (sage) {
-            if (D == 256) H3_QK(true, 256);
-            else if (D == 128) H3_QK(true, 128);
+            // (the int8 form is for heads of 64 or 128 features only)
+            if (D == 128) H3_QK(true, 128);
             else H3_QK(true, 64);
         } else {
             if (D == 256) H3_QK(false, 256);
@@ -46,8 +46,7 @@ static void prep(Ctx* c, const void* q, const void* k, const void* v, int64_t S,
             qk(k, kv_stride, kvblocks, mean, ak, sc);
             attn_v_prep_kernel<DT><<<kvblocks, 256, 0, c->stream>>>(v, S, Sp, D, __builtin_ctz((unsigned) DK), kv_stride, av);
         } else if (sage) {
-            if (D == 256) H3_KV(true, 256);
-            else if (D == 128) H3_KV(true, 128);
+            if (D == 128) H3_KV(true, 128);
             else H3_KV(true, 64);
         } else {
             if (D == 256) H3_KV(false, 256);
@@ -189,12 +188,6 @@ static int attention_one(Ctx* c, const char* fn, const void* q, const void* k, c
         if (pad) attn_kernel<SG, DD, CA, true><<<grid, 256, 0, c->stream>>>(P);               \
         else attn_kernel<SG, DD, CA, false><<<grid, 256, 0, c->stream>>>(P);                  \
     }
-#define H3_ATTN(SG, CA)                                                                        \
-    {                                                                                          \
-        if (DK == 256) H3_ATTN_D(SG, 256, CA)                                                  \
-        else if (DK == 128) H3_ATTN_D(SG, 128, CA)                                             \
-        else H3_ATTN_D(SG, 64, CA)                                                             \
-    }
     if (pp) {
         if (sage) attn_pl_kernel<true, 6><<<grid, 256, 0, c->stream>>>(P);
         else attn_pl_kernel<false, 4><<<grid, 256, 0, c->stream>>>(P);
@@ -202,13 +195,21 @@ static int attention_one(Ctx* c, const char* fn, const void* q, const void* k, c
     } else if (causal && DK <= 128 && attn_causal_groups(S, Hq, c->cus)) {
         if (DK == 128) { if (pad) attn_kernel<false, 128, true, true, 2><<<grid, 512, 0, c->stream>>>(P); else attn_kernel<false, 128, true, false, 2><<<grid, 512, 0, c->stream>>>(P); }
         else { if (pad) attn_kernel<false, 64, true, true, 2><<<grid, 512, 0, c->stream>>>(P); else attn_kernel<false, 64, true, false, 2><<<grid, 512, 0, c->stream>>>(P); }
-    } else if (causal) H3_ATTN(false, true)
-    else if (sage) {
-        // (the int8 form only at 64 or 128 features, above)
-        if (DK == 128) H3_ATTN_D(true, 128, false)
-        else H3_ATTN_D(true, 64, false)
-    } else H3_ATTN(false, false)
-#undef H3_ATTN
+    } else if (causal) {
+        if (DK == 256) H3_ATTN_D(false, 256, true)
+        else if (DK == 128) H3_ATTN_D(false, 128, true)
+        else H3_ATTN_D(false, 64, true)
+    } else if (DK == 128) {
+        // (heads of 65 to 127 features, or an out off 16-byte boundaries: the others took the wide kernel)
+        if (sage) attn_kernel<true, 128, false, true><<<grid, 256, 0, c->stream>>>(P);
+        else attn_kernel<false, 128, false, true><<<grid, 256, 0, c->stream>>>(P);
+    } else if (DK == 256) {
+        H3_ATTN_D(false, 256, false)
+    } else if (sage) {
+        H3_ATTN_D(true, 64, false)
+    } else {
+        H3_ATTN_D(false, 64, false)
+    }
 #undef H3_ATTN_D
     if (launched(fn)) return -1;
     timer.mark();

@@ -226,7 +226,7 @@ __global__ __launch_bounds__(kSkinnyThreads, 2 * skinny_per_cu(MT, NT)) void gem
             }
 }
 
-// a thread sums four values' parts in part order: 64 MT * 64 / 4 threads a tile
+// a thread sums four values' parts in part order: 64 MT * 64 NT / 4 threads a tile
 template <int MT, int NT, bool SWAP>
 __global__ __launch_bounds__(256) void skinny_merge_kernel(SkinnyArgs P) {
     constexpr int PER = 64 * MT * 64 * NT / 4;

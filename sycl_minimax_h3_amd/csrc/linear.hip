@@ -150,9 +150,12 @@ static void skinny_one(Ctx* c, const SkinnyArgs& P) {
 }
 template <int OP, bool SWAP>
 static void skinny_mt(Ctx* c, const SkinnyArgs& P, int mt, int nt) {
-#define H3_SK(MM) case MM: if (nt == 2) skinny_one<OP, MM, 2, SWAP>(c, P); else skinny_one<OP, MM, 1, SWAP>(c, P); break;
-    switch (mt) {
-        H3_SK(1) H3_SK(2) H3_SK(3) H3_SK(4)
+#define H3_SK(MM) { if (nt == 2) skinny_one<OP, MM, 2, SWAP>(c, P); else skinny_one<OP, MM, 1, SWAP>(c, P); }
+    if (mt == 1) H3_SK(1)
+    else if (SWAP || mt == 2) H3_SK(2)                           // (swapped: at most 128 rows of w)
+    else if constexpr (!SWAP) {
+        if (mt == 3) H3_SK(3)
+        else H3_SK(4)
     }
 #undef H3_SK
 }

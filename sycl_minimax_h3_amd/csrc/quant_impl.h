@@ -1121,9 +1121,9 @@ template <int XDT> int quant_launch(Ctx* c, const char* fn, const QuantArgs& A, 
     if (mode == QUANT_NORM_OUT) f |= ROW_OUTH;
     // the model's widths, one or two wavefronts a row
     if constexpr (XDT != H3S_F32) {
-        // From 8192 rows; with the checkpoints' rotation from 1024: the pair layout's rotation takes fewer instructions than the general kernel's, which shows as soon as the launch is longer than its latency
-        // (2159 rows: swiglu 14336 36.0 -> 31.3 us, x 14336 25.8 -> 20.7, norm with
-        // tables 22.2 -> 17.2; 1024 rows: 18.7 -> 14.9, 13.5 -> 9.5, 11.5 -> 9.2). Unrotated the two are alike up to 6000
+        // From 8192 rows; with the checkpoints' rotation from 1024: the pair layout's rotation takes fewer instructions than
+        // the general kernel's, which shows as soon as the launch is longer than its latency (2159 rows: swiglu 14336 36.0 ->
+        // 31.3 us, x 14336 25.8 -> 20.7, norm with tables 22.2 -> 17.2; 1024 rows: 18.7 -> 14.9, 13.5 -> 9.5, 11.5 -> 9.2). Unrotated the two are alike up to 6000
         // rows (7168 features at 2159 rows: 8.5 general, 10.4 here). The norm without tables from 2560 (1500 rows 10.4 general,
         // 10.8 here, 2159 rows 13.6, 14.0, 3071 rows 17.5, 14.5).
         const bool reg256 = A.rot == H3S_ROT_REGULAR && A.group == 256;
