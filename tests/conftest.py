@@ -51,6 +51,25 @@ def dev_wave():
 
 
 @pytest.fixture(scope="session")
+def dev_four():
+    """A context whose row quantizer takes the layouts of short inputs (four wavefronts a row at the longer rows) at every row
+    count a test reaches (a large H3S_QUANT_WAVE_MIN_ROWS)."""
+    from sycl_minimax_h3_amd import Device
+
+    old = os.environ.get("H3S_QUANT_WAVE_MIN_ROWS")
+    os.environ["H3S_QUANT_WAVE_MIN_ROWS"] = "1000000000"
+    try:
+        d = Device.open()
+    finally:
+        if old is None:
+            del os.environ["H3S_QUANT_WAVE_MIN_ROWS"]
+        else:
+            os.environ["H3S_QUANT_WAVE_MIN_ROWS"] = old
+    yield d
+    d.close()
+
+
+@pytest.fixture(scope="session")
 def dev_cus16():
     """A context that sizes its grids for 16 compute units (H3S_CUS=16): GEMMs of a few dozen tiles then make whole
     rounds of tiles (XCD renumbering and tile groups, no split along K) at sizes the oracle checks quickly."""

@@ -432,3 +432,28 @@ def test_attention_dead_keys(dev, dev_16, form, dt, L, Hq, D, dead, value):
     rel, _ = o.compare(got.ravel(), want[rows].astype(np.float32).ravel())
     # P in half, the result in dt: 2^-9 of bfloat16 (relative 2-norm 1.7e-3), under 1e-3 of half's weights
     assert rel < (3e-3 if dt == o.BF16 else 1e-3), f"relative L2 {rel:.2e}"
+
+
+@pytest.mark.parametrize("sage", [True, False])
+def test_attention_without_room_for_parts(sage):
+    """a context whose memory is taken: the split blocks' partial sums have no room, and every block runs whole"""
+    d = _open_with({"H3S_MEM_FRACTION": "0.05", **({"H3S_SAGE_MIN_S": "0"} if sage else {"H3S_ATTN": "onednn"})})
+    S, H, D = 777, 3, 128
+    W = H * D
+    q, k, v = qkv(160, S, H, D, o.BF16, W)
+    want = o.attention(q, k, v, o.BF16, S, H, D, W, out_dt=o.BF16, sage=sage)
+    want = want[0] if sage else want
+    qr, kr, vr = (ops.Rows(up(d, a, "BF16", [S, W]), 0, W, S, H, D) for a in (q, k, v))
+    out = new(d, "BF16", [S, W])
+    t = new(d, "BF16", [64, 4 * W])                              # a call of whole blocks that grows the other scratch as far
+    r = ops.Rows(t, 0, 4 * W, 64, 4 * H, D)
+    ops.attention(r, r, r, t)
+    rest = new(d, "U8", [d.mem_cap() - d.mem_used() - (1 << 20)])
+    names = [n.split("<")[0] for n, _, _ in launches(d, lambda: ops.attention(qr, kr, vr, out))]
+    check(out.to_numpy().ravel(), want, o.BF16, "whole blocks")
+    assert "attn_merge_kernel" not in names, names
+    del rest
+    names = [n.split("<")[0] for n, _, _ in launches(d, lambda: ops.attention(qr, kr, vr, out))]
+    check(out.to_numpy().ravel(), want, o.BF16, "split blocks")
+    assert "attn_merge_kernel" in names, names
+    d.close()

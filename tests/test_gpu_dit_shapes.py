@@ -43,7 +43,7 @@ def dit_rows(M):
                                                    (9, 130, False, False, o.F32)])
 @pytest.mark.parametrize("layout", ["four", "wave"])
 def test_int8_linear_dit_widths(request, layout, K, M, N, per_n, bias, out_dt):
-    dev = request.getfixturevalue("dev" if layout == "four" else "dev_wave")
+    dev = request.getfixturevalue("dev_four" if layout == "four" else "dev_wave")
     rng = np.random.default_rng(K + M + N)
     x = bf16_rows(K + M, M, K, 0.7)
     w = rng.integers(-127, 128, N * K, dtype=np.int8)
@@ -61,8 +61,8 @@ def test_int8_linear_dit_widths(request, layout, K, M, N, per_n, bias, out_dt):
 @pytest.mark.parametrize("group", [256, 0])
 @pytest.mark.parametrize("layout", ["four", "wave"])
 def test_int8_quantize_dit_widths(request, layout, K, group):
-    dev = request.getfixturevalue("dev" if layout == "four" else "dev_wave")
-    M = 8200 if K == DH else 2100                  # past the one-wavefront form's row threshold at the hidden width
+    dev = request.getfixturevalue("dev_four" if layout == "four" else "dev_wave")
+    M = 8200 if K == DH else 2100
     x = bf16_rows(K + group, M, K)
     want_q, want_s = o.quantize_act(x, o.BF16, M, K, o.ROT_REGULAR if group else o.ROT_NONE, group)
     q, s = new(dev, "I8", [M, K]), new(dev, "F32", [M])
@@ -74,7 +74,7 @@ def test_int8_quantize_dit_widths(request, layout, K, group):
 # ---- the two-chunks-a-lane (16 features) layout of the regular-256 rotation at the other widths it serves ----
 @pytest.mark.parametrize("layout", ["four", "wave"])
 def test_int8_quantize_4096_pairs(request, layout):
-    dev = request.getfixturevalue("dev" if layout == "four" else "dev_wave")
+    dev = request.getfixturevalue("dev_four" if layout == "four" else "dev_wave")
     M, K = 1025, 4096
     x = bf16_rows(90, M, K)
     want_q, want_s = o.quantize_act(x, o.BF16, M, K, o.ROT_REGULAR, 256)
@@ -157,7 +157,7 @@ def test_quant_rows_of_the_environment(dev_rows5000, kind, C, rot, group, M, wav
 
 @pytest.mark.parametrize("layout", ["four", "wave"])
 def test_swiglu_quant_8192_pairs(request, layout):
-    dev = request.getfixturevalue("dev" if layout == "four" else "dev_wave")
+    dev = request.getfixturevalue("dev_four" if layout == "four" else "dev_wave")
     M, C = 301, 8192
     x = bf16_rows(91, M, 2 * C, 4.0, heavy=False)
     xt = up(dev, x, "BF16", [M, 2 * C])
@@ -174,7 +174,7 @@ def test_swiglu_quant_8192_pairs(request, layout):
 @pytest.mark.parametrize("M,rot,group", [(9, o.ROT_REGULAR, 256), (2500, o.ROT_REGULAR, 256), (33, o.ROT_NONE, 0)])
 @pytest.mark.parametrize("layout", ["four", "wave"])
 def test_swiglu_quant_fc2_width(request, layout, M, rot, group):
-    dev = request.getfixturevalue("dev" if layout == "four" else "dev_wave")
+    dev = request.getfixturevalue("dev_four" if layout == "four" else "dev_wave")
     C = DFF
     x = bf16_rows(M + 41, M, 2 * C, 4.0, heavy=False)
     xt = up(dev, x, "BF16", [M, 2 * C])
@@ -207,7 +207,7 @@ def tiny_rows(seed, C, heavy=True):
 @pytest.mark.parametrize("K", [DH, DHEADS * DHD, DFF, 4096])
 @pytest.mark.parametrize("layout", ["four", "wave"])
 def test_int8_quantize_tiny_rows(request, layout, K):
-    dev = request.getfixturevalue("dev" if layout == "four" else "dev_wave")
+    dev = request.getfixturevalue("dev_four" if layout == "four" else "dev_wave")
     x, M = tiny_rows(K, K)
     want_q, want_s = o.quantize_act(x, o.BF16, M, K, o.ROT_REGULAR, 256)
     q, s = new(dev, "I8", [M, K]), new(dev, "F32", [M])
@@ -219,7 +219,7 @@ def test_int8_quantize_tiny_rows(request, layout, K):
 @pytest.mark.parametrize("C", [DFF, 8192])
 @pytest.mark.parametrize("layout", ["four", "wave"])
 def test_swiglu_quant_tiny_rows(request, layout, C):
-    dev = request.getfixturevalue("dev" if layout == "four" else "dev_wave")
+    dev = request.getfixturevalue("dev_four" if layout == "four" else "dev_wave")
     x, M = tiny_rows(C + 7, 2 * C, heavy=False)
     xt = up(dev, x, "BF16", [M, 2 * C])
     q, s = new(dev, "I8", [M, C]), new(dev, "F32", [M])
@@ -235,7 +235,7 @@ def test_swiglu_quant_tiny_rows(request, layout, C):
 def test_norm_quant_tiny_weight(request, layout):
     """the norm's rows are O(|w|) whatever x is: weights of 2^-62 .. 2^-75 put the rotated rows on both sides of the
     threshold"""
-    dev = request.getfixturevalue("dev" if layout == "four" else "dev_wave")
+    dev = request.getfixturevalue("dev_four" if layout == "four" else "dev_wave")
     M, C = 96, DH
     x = bf16_rows(53, M, C)
     rng = np.random.default_rng(54)
@@ -256,7 +256,7 @@ def test_norm_quant_tiny_weight(request, layout):
 @pytest.mark.parametrize("rot,group", [(o.ROT_REGULAR, 256), (o.ROT_NONE, 0)])
 @pytest.mark.parametrize("layout", ["four", "wave"])
 def test_norm_quant_dit_width(request, layout, rot, group):
-    dev = request.getfixturevalue("dev" if layout == "four" else "dev_wave")
+    dev = request.getfixturevalue("dev_four" if layout == "four" else "dev_wave")
     M, C = 16896, DH
     x = bf16_rows(51, M, C)
     rng = np.random.default_rng(52)
@@ -357,7 +357,7 @@ def test_rms_norm_mod_streamed_steps(dev_cus2, M, mod):
 @pytest.mark.parametrize("M", [1, 37, 300])
 @pytest.mark.parametrize("layout", ["four", "wave"])
 def test_rms_norm_mod_dit_width(request, layout, mod, M):
-    dev = request.getfixturevalue("dev" if layout == "four" else "dev_wave")
+    dev = request.getfixturevalue("dev_four" if layout == "four" else "dev_wave")
     C = DH
     x = bf16_rows(80 + M, M, C)
     rng = np.random.default_rng(81)

@@ -1,8 +1,8 @@
 """GPU parity of the matrix-core GEMMs whose last tiles split along K (int8: h3s_int8_gemm_dequant, h3s_int8_linear;
-16-bit: h3s_linear, h3s_linear_acc), against the oracle. The split takes rows of at least 12288 bytes; a context
-that sizes its grids for 4 compute units (H3S_CUS=4) gives small products the short last round it is for: 6 tiles
-(4 whole, 2 in 2 parts of 48 K steps) and 5 tiles (4 whole, the fifth in 4 parts, the last ending on a half step
-where K is an odd multiple of 64 bytes). The int8 parts' int32 sums are exact, so the int8 results stay bit for bit
+16-bit: h3s_linear, h3s_linear_acc) or whose tiles are lower than 256 rows, against the oracle. The split takes rows of at
+least 12288 bytes; a context that sizes its grids for 4 compute units (H3S_CUS=4) gives small products the short last
+round it is for: 6 tiles (4 whole, 2 in 2 parts of 48 K steps) and 5 tiles (4 whole, the fifth in 4 parts, the last
+ending on a half step where K is an odd multiple of 64 bytes). The cases say which tiles they reach and check it. The int8 parts' int32 sums are exact, so the int8 results stay bit for bit
 the oracle's; the 16-bit results keep the float linear's tolerance."""
 import os
 
@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as o
-from helpers import assert_bits_equal, assert_close_16, new, up
+from helpers import assert_bits_equal, assert_close_16, launches, new, up
 from sycl_minimax_h3_amd import DType, ops
 
 pytestmark = pytest.mark.gpu
@@ -36,15 +36,22 @@ def dev4():
 
 
 # (M, K, N): tiles of 256 x 256, K steps of 128 bytes
-SHAPES_I8 = [(260, 12288, 600),   # 2 x 3 tiles: 4 whole, 2 in 2 parts of 48 steps
+SHAPES_I8 = [(500, 12288, 600),   # 2 x 3 tiles: 4 whole, 2 in 2 parts of 48 steps
              (1100, 12352, 200)]  # 5 x 1: 4 whole, 1 in 4 parts; 96.5 steps, the half step in the last part
+SPLIT_BLOCKS = 8                  # of both: 4 + 2 x 2 and 4 + 1 x 4
+
+
+def check_split(got, tiles="gemm_"):
+    """the launches of a product whose last tiles are split: the tiles of 256 rows, then the merge"""
+    assert len(got) == 2 and got[0][0].startswith(tiles) and got[0][0].endswith(" 4>") and got[0][1] == SPLIT_BLOCKS, got
+    assert got[1][0].startswith("gemm_merge_kernel<"), got
 
 
 @pytest.mark.parametrize("act", [o.ACT_NONE, o.ACT_SILU])
 @pytest.mark.parametrize("per_n,bias,out_dt", [(False, False, o.BF16), (True, True, o.BF16), (True, False, o.F32),
                                                (False, True, o.F16)])
 @pytest.mark.parametrize("M,K,N", SHAPES_I8)
-def test_int8_gemm_split(dev4, M, K, N, per_n, bias, out_dt, act):
+def test_int8_gemm_split(dev4, M, K, N, per_n, bias, out_dt, act, wi=None):
     rng = np.random.default_rng(M + K + N)
     q = rng.integers(-128, 128, M * K, dtype=np.int8)
     s = rng.uniform(0.001, 0.05, M).astype(np.float32)
@@ -54,7 +61,12 @@ def test_int8_gemm_split(dev4, M, K, N, per_n, bias, out_dt, act):
     want = o.gemm_dequant(q, s, M, K, w, N, ws, b, act, out_dt)
     layer = ops.Int8Linear(up(dev4, w, "I8", [N, K]), up(dev4, ws, "F32", [ws.size]), up(dev4, b, "F32", [N]) if bias else None)
     out = new(dev4, DTS[out_dt], [M, N])
-    ops.int8_gemm_dequant(up(dev4, q, "I8", [M, K]), up(dev4, s, "F32", [M]), layer, act, out)
+    qt, st = up(dev4, q, "I8", [M, K]), up(dev4, s, "F32", [M])
+    got = launches(dev4, lambda: ops.int8_gemm_dequant(qt, st, layer, act, out))
+    if wi is None:
+        check_split(got, "gemm_i8_kernel<")
+    else:
+        assert [n.rpartition(", ")[2] for n, _, _ in got] == [f"{wi}>"] and got[0][1] == -(-M // (64 * wi)) * -(-N // 256), got
     if act == o.ACT_NONE or out_dt == o.F32:
         if act == o.ACT_NONE:
             assert_bits_equal(out.to_numpy(), want, "gemm split")
@@ -65,26 +77,26 @@ def test_int8_gemm_split(dev4, M, K, N, per_n, bias, out_dt, act):
         assert_close_16(out.to_numpy(), want, out_dt, "gemm split silu", max_frac=5e-3)
 
 
-# launches of few rounds take tiles of 192 or 128 rows (gemm_plan, for 4 compute units): (192) 2 x 3 tiles with a half step,
-# 2 x 2 whole tiles, one row of 4; (128) one row of 3 tiles, whole rows and a half step; and 256 rows with its split kept
+# launches of few rounds take tiles of 64 wi rows (gemm_plan, for 4 compute units): 192 rows, 2 x 3 tiles with a half step, 2 x 2
+# whole tiles, one row of 4, and 2 x 3 of 96 steps; 128 rows, one row of 3 tiles, whole rows and a half step, one live row
 @pytest.mark.parametrize("per_n,bias,out_dt", [(False, False, o.BF16), (True, True, o.F32), (True, False, o.F16)])
-@pytest.mark.parametrize("M,K,N", [(260, 4160, 600), (384, 4096, 500), (190, 4224, 1000), (120, 4096, 600), (128, 4160, 700), (1, 4096, 601),
-                                   (500, 12288, 600)])
-def test_int8_gemm_tile_heights(dev4, M, K, N, per_n, bias, out_dt):
-    test_int8_gemm_split(dev4, M, K, N, per_n, bias, out_dt, o.ACT_NONE)
+@pytest.mark.parametrize("wi,M,K,N", [(3, 260, 4160, 600), (3, 384, 4096, 500), (3, 190, 4224, 1000), (3, 260, 12288, 600), (2, 120, 4096, 600),
+                                      (2, 128, 4160, 700), (2, 1, 4096, 601)])
+def test_int8_gemm_tile_heights(dev4, wi, M, K, N, per_n, bias, out_dt):
+    test_int8_gemm_split(dev4, M, K, N, per_n, bias, out_dt, o.ACT_NONE, wi)
 
 
-# the same on 16-bit operands: 192 rows (3 x 2 tiles, a half step; 4 x 1), 128 rows (5 x 3), 256 rows with its split kept
+# the same on 16-bit operands: 192 rows (3 x 2 tiles, a half step; 4 x 1), 128 rows (5 x 3)
 @pytest.mark.parametrize("dt,out_dt,bias", [(o.BF16, o.BF16, True), (o.F16, o.F32, False)])
-@pytest.mark.parametrize("M,K,N", [(520, 2080, 300), (640, 2048, 200), (640, 2080, 600), (1100, 6176, 200)])
-def test_linear_tile_heights(dev4, dt, out_dt, bias, M, K, N):
-    test_linear_split(dev4, dt, out_dt, M, K, N, bias)
+@pytest.mark.parametrize("wi,M,K,N", [(3, 520, 2080, 300), (3, 640, 2048, 200), (2, 640, 2080, 600)])
+def test_linear_tile_heights(dev4, dt, out_dt, bias, wi, M, K, N):
+    test_linear_split(dev4, dt, out_dt, M, K, N, bias, wi)
 
 
 @pytest.mark.parametrize("group", [0, 256])
 def test_int8_linear_split(dev4, group):
     """h3s_int8_linear (the quantizer, then the GEMM with its last tiles split) against the oracle, bit for bit."""
-    M, K, N = 260, 12288, 600
+    M, K, N = SHAPES_I8[0]
     rng = np.random.default_rng(77 + group)
     x = o.to_bf16((0.7 * rng.standard_normal(M * K)).astype(np.float32))
     w = rng.integers(-127, 128, N * K, dtype=np.int8)
@@ -92,8 +104,9 @@ def test_int8_linear_split(dev4, group):
     b = rng.standard_normal(N).astype(np.float32)
     want = o.int8_linear(x, o.BF16, M, K, w, N, ws, b, o.BF16, group)
     layer = ops.Int8Linear(up(dev4, w, "I8", [N, K]), up(dev4, ws, "F32", [N]), up(dev4, b, "F32", [N]), group or None)
-    out = new(dev4, "BF16", [M, N])
-    layer.forward(up(dev4, x, "BF16", [M, K]), out)
+    out, xt = new(dev4, "BF16", [M, N]), up(dev4, x, "BF16", [M, K])
+    got = launches(dev4, lambda: layer.forward(xt, out))
+    check_split(got[1:], "gemm_i8_kernel<")                      # (after the quantizer)
     assert_bits_equal(out.to_numpy(), want, "int8_linear split")
 
 
@@ -114,14 +127,19 @@ def close(got, want, dt, what):
 
 
 @pytest.mark.parametrize("dt,out_dt", [(o.BF16, o.BF16), (o.BF16, o.F32), (o.F16, o.F16)])
-@pytest.mark.parametrize("M,K,N", [(260, 6144, 600), (1100, 6176, 200)])
+@pytest.mark.parametrize("M,K,N", [(600, 6144, 500), (1100, 6176, 200)])     # 3 x 2 tiles, 4 whole, 2 in 2 parts; 5 x 1 as above
 @pytest.mark.parametrize("bias", [False, True])
-def test_linear_split(dev4, dt, out_dt, M, K, N, bias):
+def test_linear_split(dev4, dt, out_dt, M, K, N, bias, wi=None):
     x, w, b = mats(200 + K, M, K, N, dt)
     want = o.linear(x, dt, M, K, w, N, b if bias else None, out_dt=out_dt)
     out = new(dev4, DTS[out_dt], [M, N])
     layer = ops.Linear(up(dev4, w, DTS[dt], [N, K]), up(dev4, b, "F32", [N]) if bias else None)
-    layer.forward(up(dev4, x, DTS[dt], [M, K]), out)
+    xt = up(dev4, x, DTS[dt], [M, K])
+    got = launches(dev4, lambda: layer.forward(xt, out))
+    if wi is None:
+        check_split(got, "gemm_f16_kernel<")
+    else:
+        assert [n.rpartition(", ")[2] for n, _, _ in got] == [f"{wi}>"] and got[0][1] == -(-M // (64 * wi)) * -(-N // 256), got
     close(out.to_numpy(), want, out_dt, "linear split")
 
 

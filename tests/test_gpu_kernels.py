@@ -244,7 +244,7 @@ def test_qk_rms_rope_dit_call(dev, rot):
                                     (o.F16, 2048)])
 @pytest.mark.parametrize("layout", ["four", "wave"])
 def test_norm_quant(request, layout, rot, group, x_dt, C):
-    dev = request.getfixturevalue("dev" if layout == "four" else "dev_wave")
+    dev = request.getfixturevalue("dev_four" if layout == "four" else "dev_wave")
     if group and C % group:
         pytest.skip("group does not divide C")
     if rot == o.ROT_SYLVESTER and group > 64 * (16 // (4 if x_dt == o.F32 else 2)):
@@ -266,7 +266,7 @@ def test_norm_quant(request, layout, rot, group, x_dt, C):
 @pytest.mark.parametrize("h_dt", [o.BF16, o.F32, o.F16])
 @pytest.mark.parametrize("layout", ["four", "wave"])
 def test_norm_quant_modulated(request, layout, tab_dt, with_rows, h_dt):
-    dev = request.getfixturevalue("dev" if layout == "four" else "dev_wave")
+    dev = request.getfixturevalue("dev_four" if layout == "four" else "dev_wave")
     M, C, R = 29, 4096, 3
     x = inputs(24, M * C, o.BF16)
     w = weight(25, C)
@@ -286,7 +286,7 @@ def test_norm_quant_modulated(request, layout, tab_dt, with_rows, h_dt):
 @pytest.mark.parametrize("layout", ["four", "wave"])
 def test_norm_quant_edge_rows(request, layout):
     """A zero row (scale 1e-30, codes 0), a constant row, huge and tiny rows, and a row count not a multiple of 4."""
-    dev = request.getfixturevalue("dev" if layout == "four" else "dev_wave")
+    dev = request.getfixturevalue("dev_four" if layout == "four" else "dev_wave")
     M, C = 6, 4096
     x = np.random.default_rng(28).standard_normal((M, C)).astype(np.float32)
     x[0] = 0.0
@@ -578,7 +578,7 @@ def test_chain_two_rows_a_block(dev, kind, C, M):
 @pytest.mark.parametrize("per_n,bias,out_dt", [(False, False, o.BF16), (True, True, o.BF16), (True, False, o.F32)])
 @pytest.mark.parametrize("layout", ["four", "wave"])
 def test_int8_linear(request, layout, M, K, N, group, per_n, bias, out_dt):
-    dev = request.getfixturevalue("dev" if layout == "four" else "dev_wave")
+    dev = request.getfixturevalue("dev_four" if layout == "four" else "dev_wave")
     if group and K % group:
         pytest.skip("group does not divide K")
     rng = np.random.default_rng(M * 7 + K + N + group)
