@@ -187,12 +187,14 @@ static SkinnyPlan skinny_plan(int64_t S, int64_t L, int64_t nk, int cus) {
 // to 16 steps); and else by the two whole times in microseconds. Here: 0.0026 a row and step, a block's end (the groups'
 // exchange, 8-byte stores) 0.76 a 64 x 64 piece and round, 3.8 for the launch. There: gemm_plan's estimate, 3.9 for the
 // launch with the short epilogue of a tile inside out, 0.035 more a live row of a tile cut at out's edge (its stores go
-// element by element), 5.5 with a merge. Operands past the 256 MB cache come at 6.5 TB/s here, by the blocks' share of the
-// CUs, and there at 5, and a step of 256, 192 or 128 rows then takes 1.75, 1.55 or 1.33 however few the blocks. Timed both
-// ways over 1 .. 512 rows against 256 .. 65536 outputs, and 513 .. 47104 against 8 .. 128, of 64 .. 14336 features (bfloat16,
-// 2099 products): the choice is 0.3 % off the faster on average, and within 5 % of it in 97 %. Always here, products of one to
-// four steps and of more outputs than fill one round had lost to the tiles: 512 rows 64 -> 28672 8.5 -> 24.1 us, 512 rows
-// 5376 -> 28672 143 -> 174, 256 rows 64 -> 5376 5.7 -> 7.9.
+// element by element), 5.5 with a merge. Weights that a model's other layers have pushed out of the caches come slower there
+// than here: a step of 256, 192 or 128 rows then takes 1.75, 1.55 or 1.33 however few the blocks (counted in full from 32
+// steps, where the weights are megabytes, and half from 8). Operands past the 256 MB cache come at 6.5 TB/s here, by the
+// blocks' share of the CUs, and at 5 there. Timed both ways over 1 .. 512 rows against 256 .. 65536 outputs, and 513 .. 47104
+// against 8 .. 128, of 64 .. 14336 features (bfloat16, 2099 products, their weights cached): the choice is 0.4 % off the faster
+// on average, and within 5 % of it in 96 %; with cold weights (189 products) within 3 % of always taking this kernel where that
+// is faster. Always here, products of one to four steps and of more outputs than fill one round had lost to the tiles: 512
+// rows 64 -> 28672 8.5 -> 24.1 us, 512 rows 5376 -> 28672 143 -> 181, 256 rows 64 -> 5376 5.7 -> 7.9.
 static bool skinny_loses(const SkinnyPlan& p, bool swap, int64_t M, int64_t N, int64_t nk, int cus) {
     if (p.parts > 1) return false;
     const int64_t round = (int64_t) cus * skinny_per_cu(p.mt, p.nt), rounds = (p.blocks + round - 1) / round;
@@ -205,13 +207,14 @@ static bool skinny_loses(const SkinnyPlan& p, bool swap, int64_t M, int64_t N, i
     const GemmPlan g = gemm_plan(M, N, nk, cus, true);
     const int64_t bm = 64 * g.wi, tm = (M + bm - 1) / bm, tn = (N + kGemmBN - 1) / kGemmBN;
     double tiles = g.us;
-    if (!cached) {
+    if (!cached || nk >= 8) {
         const double step = g.wi == 4 ? 1.75 : g.wi == 3 ? 1.55 : 1.33;
         double t = (double) ((g.main_tiles + cus - 1) / cus * nk) * step;
         if (g.split > 1)
             t += (double) ((nk + g.split - 1) / g.split) * step +
                  0.1 * (double) ((tm * tn - g.main_tiles) * g.split) * std::min(1.0, (double) M / kGemmBM);
-        tiles = std::max({tiles, t, bytes / 5e6});
+        if (cached && nk < 32) t = 0.5 * (t + tiles);
+        tiles = std::max({tiles, t, cached ? 0.0 : bytes / 5e6});
     }
     int64_t cut = 0;                                             // live rows that cut tiles store one after the other
     if (g.split == 1) {

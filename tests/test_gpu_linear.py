@@ -128,7 +128,8 @@ def test_linear_few_rows_without_room(dev):
 
 @pytest.mark.parametrize("few,M,K,N", [(True, 137, 64, 512), (False, 256, 64, 512), (False, 512, 128, 2048), (True, 400, 64, 256),
                                        (False, 400, 96, 21504), (True, 64, 128, 16384), (True, 512, 2048, 2048), (False, 47104, 64, 96),
-                                       (True, 47104, 64, 32), (True, 513, 64, 128), (False, 513, 64, 129)])
+                                       (True, 47104, 64, 32), (True, 513, 64, 128), (False, 513, 64, 129),
+                                       (True, 256, 512, 5376), (False, 512, 512, 10752), (True, 480, 2048, 10752)])
 def test_linear_few_rows_or_tiles(dev, few, M, K, N):
     """which of the two matrix-core kernels takes a product with few rows on one side (skinny_loses): few steps with whole
     256 x 256 tiles, or more than a round of blocks, go to the tiles, the others to the few-row kernel"""
