@@ -69,9 +69,10 @@ static void prep(Ctx* c, const void* q, const void* k, const void* v, int64_t S,
 }
 
 // Whether the causal form takes two key groups a block: where the launch's time is the walk of its longest blocks (few heads,
-// long rows). bfloat16, heads of 128: 8 heads 2048 tokens 48.9 -> 40.9 us, 32 heads 600 tokens 22.1 -> 20.5, 2048 tokens
-// 61.7 -> 57.7; but 64 heads 600 tokens 23.7 -> 24.7, 2048 tokens 94.5 -> 103 (the blocks fill the device: there two blocks of
-// one group a CU run without a common barrier), and 100 tokens 11.3 -> 12.4 (two tiles: nothing to share out)
+// long rows). bfloat16, heads of 128, one group a block -> two, all else alike: 8 heads 2048 tokens 48.9 -> 40.9 us, 32 heads
+// 600 tokens 22.1 -> 20.5, 2048 tokens 61.7 -> 57.7; but 64 heads 600 tokens 23.7 -> 24.7, 2048 tokens 94.5 -> 103 (the
+// blocks fill the device: there two blocks of one group a CU run without a common barrier), and 100 tokens 11.3 -> 12.4 (two
+// tiles: nothing to share out)
 static bool attn_causal_groups(int64_t L, int64_t Hq, int cus) { return L >= 512 && 8 * Hq <= cus; }
 // Which of the wide kernel's n blocks of T key tiles run whole (the first `full`), and into how many blocks of `ts`
 // consecutive tiles each of the others is split (`ns`, at most max_ns; 1: none): the least estimated time, in key tiles of a

@@ -500,7 +500,7 @@ __global__ __launch_bounds__(256 * KS, KS == 2 ? 2 : DK == 256 ? 1 : 3) void att
     int64_t h = blockIdx.x / P.nqb, qb = blockIdx.x % P.nqb;
     if constexpr (CAUSAL) {
         // the blocks with the most keys first (in the order of the rows the longest started last: 2048 tokens x 64 heads,
-        // with q read here and k and v prepared in one launch, 150 -> 95 us, 300 tokens 24.1 -> 15.3); each XCD (blocks
+        // with q read here and k and v prepared in one launch, 172 -> 113 us, 300 tokens 29.3 -> 21.3); each XCD (blocks
         // b % 8) a run of heads, which share k and v
         const int b = (int) blockIdx.x, H = (int) P.H;
         if (H % 8 == 0) {
@@ -781,16 +781,18 @@ constexpr int kScoreBiasBits = 0x4B400000;
 
 
 // ---- the wide form: heads of 128 features, no mask but the sequence's end (both forms) ----
-// Bound by the power the card allows in long sequences (the clock falls to 1.8-2.0 GHz), by the issue of each
-// wavefront's own instructions in short ones. One block = 4 wavefronts = 256 queries of one head; a wavefront owns 64 queries
-// (two groups of 32) and walks the keys 32 at a time: a fragment of K or V^T read from LDS feeds two products, half the
-// LDS reads a product of one group a wavefront, which ran at 1.80 instead of 2.0 GHz under the same power. Two blocks a CU: the
-// two wavefronts of a SIMD belong to different blocks, with no barrier between them, so one's softmax runs beside the
-// other's products. Per tile: the softmax of both groups, a barrier, then the P v products and the next tile's scores
-// back to back at a raised issue priority, with the ring's refill and the next fragments' reads between them.
-// 56 heads: 47104 tokens 44.4 -> 41.5 ms, 2159 tokens (16-bit form) 174 -> 155 us for the whole call. Others tried: three blocks a CU of one group
-// a wavefront, 14 % fewer cycles but at 1.62 GHz (43.7 ms); eight wavefronts sharing one ring, 42.4 ms, 42.2 with
-// their barriers half a tile apart; products and softmax taking turns behind barriers, 45.4 ms.
+// Bound by the power the card allows in long sequences (47104 tokens: the clock falls to 1.78 GHz, the matrix cores are busy
+// 62 % of it), by the issue of each wavefront's own instructions in short ones (2159: 1.92 GHz, 56 %). One block = 4
+// wavefronts = 256 queries of one head; a wavefront owns 64 queries (two groups of 32) and walks the keys 32 at a time: a
+// fragment of K or V^T read from LDS feeds two products, half the LDS reads a product of one group a wavefront (eight
+// wavefronts, one block a CU: 1.82 GHz, 55.5 % busy). Two blocks a CU: the two wavefronts of a SIMD belong to different
+// blocks, with no barrier between them, so one's softmax runs beside the other's products. Per tile: the softmax of both
+// groups, a barrier, then the P v products and the next tile's scores back to back at a raised issue priority, with the
+// ring's refill and the next fragments' reads between them. 56 heads, the whole call against those eight wavefronts: 47104
+// tokens 43.0 -> 40.9 ms, 16896 5.75 -> 5.30, 2159 tokens (16-bit form) 168 -> 145 us. Others tried, at 47104 tokens where
+// this form took 41.5 ms: three blocks a CU of one group a wavefront, 14 % fewer cycles but at 1.62 GHz (43.7 ms); eight
+// wavefronts sharing one ring, 42.4 ms, 42.2 with their barriers half a tile apart; products and softmax taking turns behind
+// barriers, 45.4 ms.
 // A ring of NS stages holds the key tiles; the stage of tile t - 1 is refilled with tile t + NS - 1 after the barrier
 // inside tile t's step, every wavefront issuing its share of the direct loads, which it waits for before the barrier that
 // publishes them (the one inside the step of the tile before). The ring's loads are inline asm (attn_dma16s), and the

@@ -581,14 +581,17 @@ inline void gemm_plan_split(int64_t tiles, int64_t nk, int cus, int* main_tiles,
 
 // The height of a launch's tiles (64 wi rows: 256, 192 or 128) and their split (256-row tiles only; may_split false: none).
 // 256 rows read the fewest bytes a product and run full rounds of the device fastest, but a launch of few rounds pays for
-// its last one: the estimate below, in microseconds a K step (a full round of 256 CUs; a last round's CUs also run faster the
-// fewer they are, from `least` up to a full round's, as the square of its share), is within about 8 % of the measured times
-// of the DiT's four int8 linears at 256 .. 16896 rows, and a lower tile is taken where it says 3 % or more. Measured, 256
-// rows against the choice: 7168 -> 5376 at 2159 rows 78.9 -> 75.7 us (189 tiles, 252), at 1500 82.1 -> 57.7, at 4096
-// 160 -> 142; 14336 -> 5376 at 2159 152 -> 146; 5376 -> 28672 at 300 62.4 -> 54.7, at 3000 448 -> 420. (16-bit operands
-// 5376 -> 14336, cold weights: 640 rows 123 -> 112, 768 128 -> 121, 520 115 -> 117.) A split launch's parts
-// are written and read at about 0.1 us a part of 256 live rows. Short products (below 32 steps) keep 256 rows: there the
-// epilogue, not the steps, is the time.
+// its last one: the estimate below is in microseconds a K step (a full round of 256 CUs; a last round's CUs also run faster
+// the fewer they are, from `least` up to a full round's, as the square of its share), and a lower tile is taken where it says
+// 3 % or more. Over the DiT's four int8 linears at 256 .. 16896 rows, cold weights, the height taken is within 5 % of the
+// fastest of the three. 256 rows (split where they are) against the choice, int8, cold weights: 7168 -> 5376 at 1500 rows 83.5
+// -> 71.0 us (126 tiles in 2 parts, 252 tiles), at 2159 86.5 -> 75.6 (189 tiles, 252), at 4096 171 -> 149; 14336 -> 5376 at
+// 2159 166 -> 148; 5376 -> 28672 at 256 73.1 -> 60.5, at 3000 447 -> 431; bfloat16 5376 -> 14336 at 640 rows 121 -> 107, at
+// 768 127 -> 119, but at 520 111 -> 117 (136 rows of cut tiles, whose stores go element by element; 256 rows cut 8).
+// Against split tiles it depends on where the weights are, which no size tells: bfloat16 4096 -> 4096 at 1100 rows, cached
+// weights, 62.8 split and 51.1 at 128 rows; 5376 -> 5376 at 1030 rows, cold, 85.6 and 93.6, 7168 -> 5376 at 1152 107 and 126.
+// A split launch's parts are written and read at about 0.1 us a part of 256 live rows. Short products (below 32 steps) keep
+// 256 rows: there the epilogue, not the steps, is the time.
 struct GemmPlan { int wi, main_tiles, split; double us; };   // (us: the steps' estimate)
 inline double gemm_round_us(int64_t tiles, int wi, int cus) {
     const double full = wi == 4 ? 1.75 : wi == 3 ? 1.33 : 1.0, least = wi == 4 ? 1.05 : wi == 3 ? 0.95 : 0.82;

@@ -4,13 +4,14 @@
 // gemm_impl.h's 256 x 256 tiles give 21 tiles to 5376 rows of weights (168 blocks after the split along K, with partial
 // sums of 256 padded rows each), a block here takes 64 or 128 rows of L against all rows of the short operand (S, up to
 // 256 a block), and holds three to eight stages of both in flight.
-// A CU's direct loads arrive at 55-59 bytes a nanosecond here whatever the tile, the stages or the products beside them (a
-// copy of the kernel without its LDS reads and products ran at the same speed), so the time of a block is its rows times
-// its steps, and the launch weighs that against the partial sums (linear.hip, skinny_plan). Products with the next
+// A CU's direct loads arrive at 52-61 bytes a nanosecond here (14336 -> 5376 in one part of 84 blocks: 137, 200 and 256 rows
+// 110, 140 and 150 us) whatever the stages or the products beside them (a copy of the kernel without its LDS reads and
+// products ran at the same speed), so the time of a block is its rows times its steps, and the launch weighs that against
+// the partial sums (linear.hip, skinny_plan); the matrix cores are busy 17 % at 137 rows. Products with the next
 // step's reads between them, and S's lines loaded ahead into the XCD's L2, gave nothing.
-// bfloat16, 137 rows (cold weights): 5376 -> 5376 32.8 -> 25.5 us (16 rows: 26.0 -> 15.6; at 5 TB/s the weights take 11.6),
-// 14336 -> 5376 59.8 -> 45.0; 512 rows 5376 -> 14336 107 -> 91 us; a LoRA's first factor 7168 -> 64 at 16896 tokens 79 -> 60,
-// at 47104 183 -> 135 us.
+// bfloat16, 137 rows (cold weights): 5376 -> 5376 32.0 -> 24.3 us (16 rows: 25.8 -> 15.7; at 5 TB/s the weights take 11.6),
+// 14336 -> 5376 59.3 -> 43.4; 512 rows 5376 -> 14336 107 -> 86 us; a LoRA's first factor 7168 -> 64 at 2159 tokens 29.8 ->
+// 13.5, at 16896 78 -> 58, at 47104 182 -> 136 us.
 //
 // Block: eight wavefronts, 2 x 2 over the tile (each 32 MT rows of S x 32 of L) and two along K (each takes two of a
 // step's four 32-byte slices: half the fragment reads a wavefront, and two wavefronts a SIMD; the second group's

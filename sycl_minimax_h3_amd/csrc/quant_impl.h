@@ -1122,10 +1122,11 @@ template <int XDT> int quant_launch(Ctx* c, const char* fn, const QuantArgs& A, 
     // the model's widths, one or two wavefronts a row
     if constexpr (XDT != H3S_F32) {
         // From 8192 rows; with the checkpoints' rotation from 1024: the pair layout's rotation takes fewer instructions than
-        // the general kernel's, which shows as soon as the launch is longer than its latency (2159 rows: swiglu 14336 36.0 ->
-        // 31.3 us, x 14336 25.8 -> 20.7, norm with tables 22.2 -> 17.2; 1024 rows: 18.7 -> 14.9, 13.5 -> 9.5, 11.5 -> 9.2). Unrotated the two are alike up to 6000
-        // rows (7168 features at 2159 rows: 8.5 general, 10.4 here). The norm without tables from 2560 (1500 rows 10.4 general,
-        // 10.8 here, 2159 rows 13.6, 14.0, 3071 rows 17.5, 14.5).
+        // the general kernel's, which shows as soon as the launch is longer than its latency (1024 rows: swiglu 14336 16.5 ->
+        // 14.5 us and 8192 10.7 -> 9.5, x 14336 12.3 -> 9.1, 5376 7.2 -> 5.9 and 4096 5.6 -> 4.7, norm of 5376 with tables
+        // 11.3 -> 9.1; 2159 rows: 32.4 -> 30.4, 19.4 -> 17.6, 22.8 -> 18.9, 11.5 -> 11.5, 8.4 -> 6.9, 21.5 -> 17.8).
+        // Unrotated the two are alike up to 6000 rows (7168 features at 2159 rows: 8.5 general, 10.4 here). The norm without
+        // tables from 2560 (1500 rows 10.4 general, 10.8 here, 2159 rows 13.6, 14.0, 3071 rows 17.5, 14.5).
         const bool reg256 = A.rot == H3S_ROT_REGULAR && A.group == 256;
         if (quant_wave_model_takes(A, f) && (A.M >= c->quant_line(!reg256 ? 8192 : f == kQuantW ? 2560 : 1024) || (f & ROW_OUTH))) {
             const int r = quant_wave_model<XDT>(c, fn, A, f);
@@ -1157,11 +1158,12 @@ template <int XDT> int quant_launch(Ctx* c, const char* fn, const QuantArgs& A, 
     // rows of 2048 or 4096 features of a 16-bit type with the exact side inputs, and enough of them (8192) to give every
     // wavefront several rows: one wavefront a row (fewer rows: four wavefronts share each, which shortens a short launch).
     // The norm without a table row per token needs no persistent blocks and pays from 3072 (4096 features, weight only: 3000
-    // rows 11.3 -> 9.5 us, 4096 rows 14.8 -> 12.7, one table row 18.9 -> 14.0; 2159 rows 9.0 against 9.2); with a table row per
-    // token 4096 rows take 19.9 general, 20.9 here. The regular rotation, and Sylvester groups other than 128, cost this layout
-    // more: at 4096 features the norm without tables takes longer up to 8192 rows (group 256 at 3072 rows 12.5 general, 14.3
-    // here; group 64 at 6000 rows 19.1, 21.4; Sylvester groups of 64 at 5000 rows 15.7, 16.4), and with a table or 2048 features
-    // the two of the regular rotation cross between 3072 rows (2048 features 9.1, 10.1) and 4096 (12.1, 10.3).
+    // rows 11.3 -> 9.5 us, 4096 rows 14.8 -> 12.7, one table row 18.9 -> 14.0; 2159 rows 9.0 against 9.2; 2048 features at
+    // 3072 rows 6.3 -> 5.2, one table row 7.4 -> 6.3); with a table row per token 4096 rows take 19.9 general, 20.9 here. The
+    // regular rotation, and Sylvester groups other than 128, cost this layout more: at 4096 features the norm without tables
+    // takes longer up to 8192 rows (group 256 at 3072 rows 12.5 general, 14.3 here; group 64 at 6000 rows 19.1, 21.4;
+    // Sylvester groups of 64 at 5000 rows 15.7, 16.4), and with a table or 2048 features the two of the regular rotation
+    // cross between 3072 rows (2048 features 9.1, 10.1) and 4096 (12.1, 10.3).
     if constexpr (XDT != H3S_F32) {
         const bool costly = A.rot == H3S_ROT_REGULAR || (A.rot == H3S_ROT_SYLVESTER && A.group != 128), tab = (f & ROW_TAB) != 0;
         const int64_t line = f == kQuantRaw || (tab && A.rows) || (costly && A.C == 4096 && !tab) ? 8192

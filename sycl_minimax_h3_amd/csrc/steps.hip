@@ -7,17 +7,17 @@
 
 namespace h3 {
 
-// out[ci][(r m + mi) C + i] = b[o] + sum_k fl(w[o, k] t[r, k]), o = mi 6 C + ci C + i: the sum in k order from -0.0
-// in float32 (dit.rs:163-170, Rust's f32 Sum), one multiply and one add a term (no fused multiply-add). Bound by the
-// read of w. A wavefront takes 64 consecutive o and NR timestep rows at once (w is read once for them; blockIdx.y counts the
-// groups of NR rows, the last one's missing rows repeating the last row, not stored); a tile of 64 o
-// x 32 k goes through registers to LDS in 16-byte pieces that cover whole 128-byte lines, two tiles in flight while
-// the one before is summed, and each lane runs its own o's NR sums (t[r, k] is a scalar operand). The LDS rows are 36
-// floats apart, so 16 lanes' 16-byte reads touch every bank once. VEC = 1 (rows that are not whole 16-byte pieces)
-// loads single floats the same way. 96768 x 256 floats with 2 timesteps, and the
-// rotations of 2159 tokens: 185.6 -> 22.6 us (the tables alone were 152, 64 dependent row loads a tile and w read once a
-// timestep; the 101 MB take 20 us at the rate of a large copy). All groups in one launch: with few outputs and many timesteps
-// a launch a group leaves the device idle (R = 1000, 384 x 256 floats: 3251 us, 99 with one launch of a row a block, 17.6 here).
+// out[ci][(r m + mi) C + i] = b[o] + sum_k fl(w[o, k] t[r, k]), o = mi 6 C + ci C + i: the sum in k order from -0.0 in
+// float32 (dit.rs:163-170, Rust's f32 Sum), one multiply and one add a term (no fused multiply-add). Bound by the read of w.
+// A wavefront takes 64 consecutive o and NR timestep rows at once (w is read once for them; blockIdx.y counts the groups of
+// NR rows, the last one's missing rows repeating the last row, not stored); a tile of 64 o x 32 k goes through registers to
+// LDS in 16-byte pieces that cover whole 128-byte lines, two tiles in flight while the one before is summed, and each lane
+// runs its own o's NR sums (t[r, k] is a scalar operand). The LDS rows are 36 floats apart, so 16 lanes' 16-byte reads touch
+// every bank once. VEC = 1 (rows that are not whole 16-byte pieces) loads single floats the same way. 96768 x 256 floats with
+// 2 timesteps, and the rotations of 2159 tokens: 185.6 -> 22.6 us (the tables alone 153 -> 20.5: 64 dependent row loads a
+// tile and w read once a timestep; the 101 MB take 20 us at the rate of a large copy). All groups in one launch: with few
+// outputs and many timesteps a launch a group leaves the device idle (R = 1000, 384 x 256 floats: 3251 us, 99 with one launch
+// of a row a block, 17.6 here).
 constexpr int kTabK = 32, kTabStride = kTabK + 4;
 template <int NR, int VEC>
 __global__ __launch_bounds__(64) void adaln_tables_kernel(const float* __restrict__ w, const float* __restrict__ b,
