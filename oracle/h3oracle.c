@@ -1,6 +1,6 @@
 /* h3oracle.c - CPU restatement of the reference's per-token layer arithmetic (see h3oracle.h).
  *
- * TEST INFRASTRUCTURE ONLY: the checker the GPU library is compared against, never part of the product path.
+ * TEST INFRASTRUCTURE ONLY: what the GPU library is compared against, never part of the product path.
  * Build with -ffp-contract=off (oracle/Makefile): every rounding step below is the one written.
  */
 #include "h3oracle.h"

@@ -1,6 +1,6 @@
 /* h3oracle.h - CPU restatement of the reference's per-token layer arithmetic.
  *
- * TEST INFRASTRUCTURE ONLY. This library is the checker: the tests, the smoke check and the CPU-baseline leg of the
+ * TEST INFRASTRUCTURE ONLY. This library is the oracle: the tests, the smoke check and the CPU-baseline leg of the
  * benchmark load it to compute what the GPU library must produce. Nothing in the product path (libh3hip.so and the
  * sycl_minimax_h3_amd package) links, loads or calls it.
  *

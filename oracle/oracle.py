@@ -1,6 +1,6 @@
 """ctypes binding of the CPU oracle (oracle/libh3oracle.so).
 
-TEST INFRASTRUCTURE ONLY: the checker. Only tests/, ``__graft_entry__.smoke()`` and bench.py's ``cpu_baseline`` leg
+TEST INFRASTRUCTURE ONLY. Only tests/, ``__graft_entry__.smoke()`` and bench.py's ``cpu_baseline`` leg
 import this module; the product (libh3hip.so, the ``sycl_minimax_h3_amd`` package) never does.
 
 Arrays are numpy; 16-bit floats travel as ``uint16`` bit patterns (bf16 or f16 per the dtype code), as the reference
